@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace adi_hip {
 namespace {
@@ -637,139 +638,205 @@ __global__ __launch_bounds__(256) void k_conv_history(const float *qkv, uint32_t
     }
 }
 
-constexpr uint32_t kDeltaTokens = 1024;  // tokens of one k_gated_delta launch, at most
+constexpr uint32_t kDeltaTokens = 1024;  // tokens of one k_gated_delta_chunk launch, at most
 
-// gated_delta_head (src/executor.cpp:121-155) for state rows [16 y, 16 y +
-// 16) of value head x over `count` tokens in order: each wave keeps four
-// rows in registers through them, a lane holding two of a row's 128 values
-// (src/simd.cpp:108-127); the state is read and written once.
-template <uint32_t WAVES>
-__device__ __forceinline__ void gated_delta_rows_of_head(const float *convolved, const float *alpha,
-                                                         const float *beta,
-                                                         const uint16_t *alpha_bias,
-                                                         const uint16_t *a_log, uint32_t count,
-                                                         float *recurrent, float *output) {
-#pragma clang fp contract(off)
-    constexpr uint32_t kRows = kDeltaRows / WAVES;  // rows of a wave
+// Sums of a and b over each 16-lane row of the wave, the two rotations of a
+// step side by side (each fills the other's wait); every lane of the row gets
+// the same bits (a rotation adds the same two partial sums in either order).
+__device__ __forceinline__ void row16_sums(float &a, float &b) {
+    const auto step = [&](auto control) {
+        const auto rotated = [](float x) {
+            return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(
+                static_cast<int>(__float_as_uint(x)), decltype(control)::value, 0xF, 0xF, true)));
+        };
+        a += rotated(a);
+        b += rotated(b);
+    };
+    step(std::integral_constant<int, 0x128>{});  // row_ror:8
+    step(std::integral_constant<int, 0x124>{});  // row_ror:4
+    step(std::integral_constant<int, 0x122>{});  // row_ror:2
+    step(std::integral_constant<int, 0x121>{});  // row_ror:1
+}
+
+// gated_delta_head over a chunk of tokens in order: block (value head, 16
+// state rows), wave w its rows 4 w .. 4 w + 3, sixteen lanes a row, lane j of
+// them columns 4 j .. 4 j + 3 and 64 + 4 j .. 64 + 4 j + 3. What bounds it is
+// the chain from one token's state to the next (dot, reduction, update), so
+// the chip's 4096 rows are spread to one wave a SIMD, with a reduction of four
+// row rotations over eight values a lane: 60 vector instructions a token for
+// four rows. One wave a row (two values a lane, six cross-lane steps, two of
+// them row swaps, four waves a SIMD) took 230 us for 512 tokens, this takes
+// 80. The block's query, key and value entries of sixteen tokens are loaded
+// while the sixteen before run, and pass through LDS (one barrier per
+// sixteen), from where each token's are read while the one before runs (read
+// at their use: 101 us). Lane j keeps token j's attended value, so sixteen
+// tokens go out in one store.
+__global__ __launch_bounds__(256, 1) void k_gated_delta_chunk(const float *convolved, const float *alpha,
+                                                              const float *beta, const uint16_t *alpha_bias,
+                                                              const uint16_t *a_log, uint32_t count,
+                                                              float *recurrent, float *output) {
+    constexpr uint32_t kStep = 16;  // tokens a stage
+    __shared__ float2 token_gates[kDeltaTokens];  // decay, beta
+    __shared__ __align__(16) float4 qk_lds[2][kStep][2 * kLinearHead / 4];  // query, then key
+    __shared__ float v_lds[2][kStep][kDeltaRows];
     const uint32_t h = blockIdx.x;
     const uint32_t kh = h / (kValueHeads / kKeyHeads);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t row0 = blockIdx.y * kDeltaRows + wave * kRows;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    const uint32_t j = lane & 15u, local_row = wave * 4u + (lane >> 4);
+    const uint32_t row = blockIdx.y * kDeltaRows + local_row;
+    // (the state's alignment is 8 bytes)
+    float2 *state = reinterpret_cast<float2 *>(recurrent + (static_cast<size_t>(h) * kLinearHead + row) * kLinearHead);
+    const float2 a = state[2u * j], b = state[2u * j + 1u], c = state[32u + 2u * j], d = state[33u + 2u * j];
+    float4 s0 = make_float4(a.x, a.y, b.x, b.y), s1 = make_float4(c.x, c.y, d.x, d.y);
+    // thread t stages float4 t % 64 (query 0-31, key 32-63) of tokens
+    // t / 64 + 4 i, and the value entry of token t / 16, row t % 16; a token
+    // past the chunk reloads the last one
+    const float4 *qk_from = reinterpret_cast<const float4 *>(
+        convolved + ((t & 63u) < 32u ? static_cast<size_t>(kh) * kLinearHead
+                                     : kQkSize + static_cast<size_t>(kh) * kLinearHead));
+    const float *v_from = convolved + 2u * kQkSize + static_cast<size_t>(h) * kLinearHead +
+                          blockIdx.y * kDeltaRows + (t & 15u);
+    struct Stage {
+        float4 qk0, qk1, qk2, qk3;
+        float v;
+    };
+    const auto load_stage = [&](uint32_t b0) {
+        const auto qk = [&](uint32_t i) {
+            const uint32_t at = min(b0 + (t >> 6) + 4u * i, count - 1u);
+            return qk_from[static_cast<size_t>(at) * (kChannels / 4u) + (t & 31u)];
+        };
+        return Stage{qk(0), qk(1), qk(2), qk(3),
+                     v_from[static_cast<size_t>(min(b0 + (t >> 4), count - 1u)) * kChannels]};
+    };
+    const auto store_stage = [&](uint32_t slot, const Stage &in) {
+        qk_lds[slot][t >> 6][t & 63u] = in.qk0;
+        qk_lds[slot][(t >> 6) + 4u][t & 63u] = in.qk1;
+        qk_lds[slot][(t >> 6) + 8u][t & 63u] = in.qk2;
+        qk_lds[slot][(t >> 6) + 12u][t & 63u] = in.qk3;
+        v_lds[slot][t >> 4][t & 15u] = in.v;
+    };
+    const Stage first = load_stage(0);
     const float bias = bf16_bits_to_float(alpha_bias[h]);
     const float rate = expf(bf16_bits_to_float(a_log[h]));
-    const float output_scale = 1.0f / sqrtf(static_cast<float>(kLinearHead));
-    float2 *state = reinterpret_cast<float2 *>(
-        recurrent + (static_cast<size_t>(h) * kLinearHead + row0) * kLinearHead);
-    float2 s[kRows];
-#pragma unroll
-    for (uint32_t j = 0; j < kRows; ++j) {
-        s[j] = state[j * (kLinearHead / 2u) + lane];
-    }
-    // every token's decay and beta gate of the head, one thread a token
-    // (count <= kDeltaTokens), so the rows' loop does not wait on them
-    __shared__ float token_decay[kDeltaTokens], token_beta[kDeltaTokens];
-    for (uint32_t b = threadIdx.x; b < count; b += blockDim.x) {
-        token_beta[b] = sigmoid_of(beta[static_cast<size_t>(b) * kValueHeads + h]);
-        const float biased = alpha[static_cast<size_t>(b) * kValueHeads + h] + bias;
+    for (uint32_t at = t; at < count; at += 256u) {
+        const float biased = alpha[static_cast<size_t>(at) * kValueHeads + h] + bias;
         const float softplus = biased > 20.0f ? biased : log1pf(expf(biased));
-        token_decay[b] = expf(-rate * softplus);
+        token_gates[at] = make_float2(expf(-rate * softplus),
+                                      sigmoid_of(beta[static_cast<size_t>(at) * kValueHeads + h]));
     }
-    __syncthreads();
-    // a token's inputs, loaded kAhead tokens before its update (a ring of
-    // registers; a load past the last token reloads the last, unused)
-    struct TokenIn {
-        float2 q, k;
-        float v[kRows];
-    };
-    const auto load_token = [&](uint32_t b, TokenIn &in) {
-        const float *token = convolved + static_cast<size_t>(b) * kChannels;
-        in.q = reinterpret_cast<const float2 *>(token + static_cast<size_t>(kh) * kLinearHead)[lane];
-        in.k = reinterpret_cast<const float2 *>(token + kQkSize + static_cast<size_t>(kh) * kLinearHead)[lane];
-        const float *v = token + 2u * kQkSize + static_cast<size_t>(h) * kLinearHead + row0;
+    const float output_scale = 1.0f / sqrtf(static_cast<float>(kLinearHead));
+    store_stage(0, first);
+    uint32_t slot = 0;
+    for (uint32_t b0 = 0; b0 < count; b0 += kStep, slot ^= 1u) {
+        // the barrier also frees the other slot: its tokens ran before it
+        __syncthreads();
+        const Stage ahead = load_stage(b0 + kStep);
+        float kept = 0.0f;
+        const uint32_t tokens = min(kStep, count - b0);
+        struct TokenIn {
+            float4 q0, q1, k0, k1;
+            float2 gates;
+            float v;
+        };
+        const auto read = [&](uint32_t u) {
+            return TokenIn{qk_lds[slot][u][j], qk_lds[slot][u][16u + j], qk_lds[slot][u][32u + j],
+                           qk_lds[slot][u][48u + j], token_gates[b0 + u], v_lds[slot][u][local_row]};
+        };
+        const auto dot = [&](const float4 &x, const float4 &y) {
+            return fmaf(s0.w, x.w, fmaf(s0.z, x.z, fmaf(s0.y, x.y, s0.x * x.x))) +
+                   fmaf(s1.w, y.w, fmaf(s1.z, y.z, fmaf(s1.y, y.y, s1.x * y.x)));
+        };
+        // token u's attended value is summed beside token u + 1's prediction
+        float attended = 0.0f;
+        const auto update = [&](uint32_t u, const TokenIn &in) {
+            float prediction = dot(in.k0, in.k1);
+            row16_sums(prediction, attended);
+            kept = j + 1u == u ? attended : kept;
+            const float decay = in.gates.x;
+            const float delta = (in.v - prediction * decay) * in.gates.y;
+            s0.x = fmaf(s0.x, decay, in.k0.x * delta);
+            s0.y = fmaf(s0.y, decay, in.k0.y * delta);
+            s0.z = fmaf(s0.z, decay, in.k0.z * delta);
+            s0.w = fmaf(s0.w, decay, in.k0.w * delta);
+            s1.x = fmaf(s1.x, decay, in.k1.x * delta);
+            s1.y = fmaf(s1.y, decay, in.k1.y * delta);
+            s1.z = fmaf(s1.z, decay, in.k1.z * delta);
+            s1.w = fmaf(s1.w, decay, in.k1.w * delta);
+            attended = dot(in.q0, in.q1);
+        };
+        // each token's entries are read from LDS while the one before runs
+        TokenIn in = read(0);
+        if (tokens == kStep) {
 #pragma unroll
-        for (uint32_t j = 0; j < kRows; ++j) {
-            in.v[j] = v[j];
-        }
-    };
-    const auto update = [&](uint32_t b, const TokenIn &in) {
-        const float beta_value = token_beta[b];
-        const float decay = token_decay[b];
-        // the rows' chains are independent: one block of code, one store
-        float attended[kRows];
-#pragma unroll
-        for (uint32_t j = 0; j < kRows; ++j) {
-            s[j].x *= decay;
-            s[j].y *= decay;
-            const float prediction = wave_sum(s[j].x * in.k.x + s[j].y * in.k.y);
-            const float delta = (in.v[j] - prediction) * beta_value;
-            s[j].x += in.k.x * delta;
-            s[j].y += in.k.y * delta;
-            attended[j] = wave_sum(s[j].x * in.q.x + s[j].y * in.q.y) * output_scale;
-        }
-        if (lane == 0) {
-            float *dst = output + static_cast<size_t>(b) * kValueSize + static_cast<size_t>(h) * kLinearHead + row0;
-            if constexpr (kRows == 4) {
-                *reinterpret_cast<float4 *>(dst) = make_float4(attended[0], attended[1], attended[2], attended[3]);
-            } else if constexpr (kRows == 2) {
-                *reinterpret_cast<float2 *>(dst) = make_float2(attended[0], attended[1]);
-            } else {
-                static_assert(kRows == 1, "one, two or four rows a wave");
-                dst[0] = attended[0];
+            for (uint32_t u = 0; u < kStep; ++u) {
+                const TokenIn next = read(u + 1u < kStep ? u + 1u : u);
+                __builtin_amdgcn_sched_barrier(0);
+                update(u, in);
+                in = next;
+            }
+        } else {
+            for (uint32_t u = 0; u < tokens; ++u) {
+                update(u, read(u));
             }
         }
-    };
-    // ring slot u holds token b0 + u; each slot is refilled (kAhead tokens
-    // on) right after its token's update, in whole blocks of kAhead tokens
-    // with every slot index a constant, so no register of a load in flight
-    // is ever copied
-    constexpr uint32_t kAhead = 8;
-    TokenIn ring[kAhead];
-#pragma unroll
-    for (uint32_t u = 0; u < kAhead; ++u) {
-        load_token(u < count ? u : count - 1u, ring[u]);
-    }
-    uint32_t b0 = 0;
-    for (; b0 + kAhead <= count; b0 += kAhead) {
-#pragma unroll
-        for (uint32_t u = 0; u < kAhead; ++u) {
-            update(b0 + u, ring[u]);
-            const uint32_t next = b0 + u + kAhead;
-            load_token(next < count ? next : count - 1u, ring[u]);
+        float unused = 0.0f;
+        row16_sums(attended, unused);
+        kept = j + 1u == tokens ? attended : kept;
+        kept *= output_scale;
+        if (j < tokens) {
+            output[static_cast<size_t>(b0 + j) * kValueSize + static_cast<size_t>(h) * kLinearHead + row] = kept;
         }
+        store_stage(slot ^ 1u, ahead);
     }
-#pragma unroll
-    for (uint32_t u = 0; u < kAhead; ++u) {
-        if (b0 + u < count) {
-            update(b0 + u, ring[u]);
-        }
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < kRows; ++j) {
-        state[j * (kLinearHead / 2u) + lane] = s[j];
-    }
+    state[2u * j] = make_float2(s0.x, s0.y);
+    state[2u * j + 1u] = make_float2(s0.z, s0.w);
+    state[32u + 2u * j] = make_float2(s1.x, s1.y);
+    state[33u + 2u * j] = make_float2(s1.z, s1.w);
 }
 
-// Block (value head, row block) over the chunk's `count` tokens: sixteen
-// waves of one row (four waves a SIMD, each hiding the others' reductions).
-__global__ __launch_bounds__(1024) void k_gated_delta(const float *convolved, const float *alpha,
-                                                     const float *beta, const uint16_t *alpha_bias,
-                                                     const uint16_t *a_log, uint32_t count,
-                                                     float *recurrent, float *output) {
-    gated_delta_rows_of_head<16>(convolved, alpha, beta, alpha_bias, a_log, count, recurrent, output);
-}
-
-// Block (value head, row block, r): one token of sequence r with its own
-// recurrent state.
+// gated_delta_head (src/executor.cpp:121-155) for one token of sequence r:
+// block (value head, row block, r), a wave four of the block's 16 state rows,
+// a lane two of a row's 128 values (src/simd.cpp:108-127).
 __global__ __launch_bounds__(256) void k_gated_delta_rows(const float *convolved,
                                                           const float *alpha, const float *beta,
                                                           const uint16_t *alpha_bias,
                                                           const uint16_t *a_log, LinearRows rows,
                                                           float *output) {
-    const uint32_t r = blockIdx.z;
-    gated_delta_rows_of_head<4>(convolved + static_cast<size_t>(r) * kChannels,
-                             alpha + static_cast<size_t>(r) * kValueHeads,
-                             beta + static_cast<size_t>(r) * kValueHeads, alpha_bias, a_log, 1,
-                             rows.recurrent[r], output + static_cast<size_t>(r) * kValueSize);
+#pragma clang fp contract(off)
+    constexpr uint32_t kRows = kDeltaRows / 4u;  // rows of a wave
+    const uint32_t h = blockIdx.x, r = blockIdx.z;
+    const uint32_t kh = h / (kValueHeads / kKeyHeads);
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t row0 = blockIdx.y * kDeltaRows + wave * kRows;
+    const float *token = convolved + static_cast<size_t>(r) * kChannels;
+    float2 *state = reinterpret_cast<float2 *>(rows.recurrent[r] +
+                                               (static_cast<size_t>(h) * kLinearHead + row0) * kLinearHead);
+    const float2 q = reinterpret_cast<const float2 *>(token + static_cast<size_t>(kh) * kLinearHead)[lane];
+    const float2 k = reinterpret_cast<const float2 *>(token + kQkSize + static_cast<size_t>(kh) * kLinearHead)[lane];
+    const float4 v = *reinterpret_cast<const float4 *>(token + 2u * kQkSize + static_cast<size_t>(h) * kLinearHead + row0);
+    const float value[kRows] = {v.x, v.y, v.z, v.w};
+    const float beta_value = sigmoid_of(beta[static_cast<size_t>(r) * kValueHeads + h]);
+    const float biased = alpha[static_cast<size_t>(r) * kValueHeads + h] + bf16_bits_to_float(alpha_bias[h]);
+    const float softplus = biased > 20.0f ? biased : log1pf(expf(biased));
+    const float decay = expf(-expf(bf16_bits_to_float(a_log[h])) * softplus);
+    const float output_scale = 1.0f / sqrtf(static_cast<float>(kLinearHead));
+    float attended[kRows];
+#pragma unroll
+    for (uint32_t j = 0; j < kRows; ++j) {
+        float2 s = state[j * (kLinearHead / 2u) + lane];
+        s.x *= decay;
+        s.y *= decay;
+        const float prediction = wave_sum(s.x * k.x + s.y * k.y);
+        const float delta = (value[j] - prediction) * beta_value;
+        s.x += k.x * delta;
+        s.y += k.y * delta;
+        attended[j] = wave_sum(s.x * q.x + s.y * q.y) * output_scale;
+        state[j * (kLinearHead / 2u) + lane] = s;
+    }
+    if (lane == 0) {
+        *reinterpret_cast<float4 *>(output + static_cast<size_t>(r) * kValueSize + static_cast<size_t>(h) * kLinearHead +
+                                    row0) = make_float4(attended[0], attended[1], attended[2], attended[3]);
+    }
 }
 
 // The causal convolution and SiLU of channel c for one token whose three
@@ -1262,10 +1329,18 @@ void linear_attention_chunk(adi_hip_context *ctx, const adi_hip_linear_attention
         launch(ctx, "linear_conv_history", k_conv_history, dim3(kChannels / 256), dim3(256), 0,
                static_cast<const float *>(qkv), count, convolution_state);
     }
+    const dim3 delta_grid(kValueHeads, kLinearHead / kDeltaRows);
+    if (count == 1) {  // the decode step's bits
+        LinearRows table{};
+        table.recurrent[0] = recurrent_state;
+        launch(ctx, "gated_delta", k_gated_delta_rows, delta_grid, dim3(256), 0, static_cast<const float *>(convolved),
+               static_cast<const float *>(alpha), static_cast<const float *>(beta), L->alpha_bias, L->a_log, table,
+               recurrent_output);
+    }
     // at most kDeltaTokens tokens a launch; the state carries over in order
-    for (uint32_t b0 = 0; b0 < count; b0 += kDeltaTokens) {
+    for (uint32_t b0 = 0; count > 1 && b0 < count; b0 += kDeltaTokens) {
         const uint32_t n = count - b0 < kDeltaTokens ? count - b0 : kDeltaTokens;
-        launch(ctx, "gated_delta", k_gated_delta, dim3(kValueHeads, kLinearHead / kDeltaRows), dim3(1024), 0,
+        launch(ctx, "gated_delta", k_gated_delta_chunk, delta_grid, dim3(256), 0,
                static_cast<const float *>(convolved + static_cast<size_t>(b0) * kChannels),
                static_cast<const float *>(alpha + static_cast<size_t>(b0) * kValueHeads),
                static_cast<const float *>(beta + static_cast<size_t>(b0) * kValueHeads), L->alpha_bias, L->a_log,

@@ -76,6 +76,29 @@ def test_linear_attention_prefill(gpu, oracle, tluts):
         close(drec.cpu().numpy(), rec, "recurrent state")
 
 
+@pytest.mark.parametrize("count", [2, 15, 16, 17, 33, 1025])
+def test_delta_chunk_edges(gpu, oracle, tluts, count):
+    """The delta rule's chunk kernel at the edges of its sixteen-token stages
+    and of its 1024-token launches, from a nonzero state: a dot of 128 products
+    in another order differs by at most 128 * 2^-24 = 8e-6 of its magnitudes,
+    and the decay keeps an error for a few tokens only, so 1e-4 of the largest
+    value bounds outputs and state."""
+    rng = syn.rng_for(65, count)
+    layer = syn.linear_attention(rng, HIDDEN, tluts[1])
+    d = hip.upload_linear_attention(gpu, layer, gpu.ne_codebook(tluts[1]))
+    held = po.LinearAttentionStruct(layer)
+    conv = rng.normal(0.0, 1.0, 8192 * 3).astype(np.float32)
+    rec = rng.normal(0.0, 0.05, 32 * 128 * 128).astype(np.float32)
+    dconv, drec = dev(conv), dev(rec)
+    x = syn.rms_normalized(syn.hidden_states(rng, count, HIDDEN))
+    out = torch.empty((count, HIDDEN), dtype=torch.float32, device="cuda")
+    hip.linear_attention_prefill(gpu, d, count, dev(x), out, dconv, drec)
+    want = np.stack([po.linear_attention_forward(oracle, held, x[b], conv, rec, isa=16)
+                     for b in range(count)])
+    assert max_rel_error(out.cpu().numpy(), want) <= 1e-4
+    assert np.max(np.abs(drec.cpu().numpy() - rec)) <= 1e-4 * np.max(np.abs(rec))
+
+
 @pytest.mark.parametrize("full", [False, True])
 def test_prefill_layer(gpu, oracle, tluts, full):
     rng = syn.rng_for(63, int(full))

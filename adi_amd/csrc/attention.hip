@@ -17,6 +17,7 @@
 //               over its share of the history, one wave per token stream,
 //               and merges its four waves
 //   combine     per head: merge the splits, times sigmoid(gate)
+//   A long chunk's partial runs on the matrix cores (attention_chunk.hip).
 // Linear attention, after the projections:
 //   conv        per 128-channel group: the width-4 causal convolution, SiLU,
 //               the state shift, and the L2 norm of the query and key heads
@@ -36,13 +37,8 @@
 namespace adi_hip {
 namespace {
 
-constexpr uint32_t kQueryHeads = 16;
-constexpr uint32_t kKvHeads = 2;
-constexpr uint32_t kHeadSize = 256;
 constexpr uint32_t kQueryStride = 2 * kHeadSize;  // query then gate, per head
 constexpr uint32_t kRopeHalf = 32;
-constexpr uint32_t kMaxSplits = 64;
-constexpr uint32_t kPartialStride = kHeadSize + 2;  // acc[256], maximum, denominator
 
 constexpr uint32_t kKeyHeads = 16;
 constexpr uint32_t kValueHeads = 32;
@@ -117,16 +113,6 @@ struct RopeDivisors {
     float divisor[kRopeHalf];
 };
 
-__device__ __forceinline__ float wave_sum(float v) {
-    v += lane_xor<1>(v);
-    v += lane_xor<2>(v);
-    v += lane_xor<4>(v);
-    v += lane_xor<8>(v);
-    v += lane_xor<16>(v);
-    v += lane_xor<32>(v);
-    return v;
-}
-
 // Sum over the block (blockDim.x a multiple of 64, at most 1024); every
 // thread receives it. `partial` holds 16 floats.
 __device__ __forceinline__ float block_sum(float v, float *partial) {
@@ -145,7 +131,6 @@ __device__ __forceinline__ float block_sum(float v, float *partial) {
 }
 
 __device__ __forceinline__ float silu_of(float v) { return v / (1.0f + expf(-v)); }
-__device__ __forceinline__ float sigmoid_of(float v) { return 1.0f / (1.0f + expf(-v)); }
 
 // normalize_head then apply_rope (src/executor.cpp:25-41, 60-72, 376-390)
 // of one 256-value head by a block of kHeadSize threads: RMS norm with
@@ -239,28 +224,6 @@ __global__ __launch_bounds__(kHeadSize) void k_norm_rope_rows(float *query_gate,
                        rows.keys[r] + entry + kv * kHeadSize, key_norm, cosine, sine, partial,
                        head);
     }
-}
-
-// update_online_softmax (src/attention.cpp:15-35) on a lane's four values.
-__device__ __forceinline__ void online_step(float score, float4 value, float &maximum,
-                                            float &denominator, float4 &acc) {
-#pragma clang fp contract(off)
-    if (score <= maximum) {
-        const float weight = expf(score - maximum);
-        denominator += weight;
-        acc.x += value.x * weight;
-        acc.y += value.y * weight;
-        acc.z += value.z * weight;
-        acc.w += value.w * weight;
-        return;
-    }
-    const float previous = expf(maximum - score);
-    denominator = denominator * previous + 1.0f;
-    acc.x = acc.x * previous + value.x;
-    acc.y = acc.y * previous + value.y;
-    acc.z = acc.z * previous + value.z;
-    acc.w = acc.w * previous + value.w;
-    maximum = score;
 }
 
 // Block (query head, split) of one token's query row: cache entries
@@ -1216,20 +1179,25 @@ void full_attention_chunk(adi_hip_context *ctx, const adi_hip_full_attention *L,
             "attention caches must be 16-byte aligned");
     auto &ws = ctx->layer_workspace;
     ws.used = 0;
+    const size_t fixed = Workspace::round(size_t(count) * kQueryHeads * kQueryStride * 4) +
+                         Workspace::round(size_t(count) * kQueryHeads * kHeadSize * 4);
+    const bool matrix = attention_chunk_takes(position, count);
     // splits of the history for the chunk's last token; a chunk's many tokens
     // already give blocks enough, so they split less
     const uint32_t last = position + count;
     const uint32_t cap = kMaxSplits / count > 0 ? kMaxSplits / count : 1u;
     uint32_t splits = ceil_div(last, 32);
     splits = splits < 1 ? 1 : (splits > cap ? cap : splits);
-    const uint32_t chunk = ceil_div(last, splits);
+    uint32_t chunk = ceil_div(last, splits);
     splits = ceil_div(last, chunk);
-    ws.ensure(Workspace::round(size_t(count) * kQueryHeads * kQueryStride * 4) +
-              Workspace::round(size_t(count) * kQueryHeads * kHeadSize * 4) +
-              Workspace::round(size_t(count) * kQueryHeads * splits * kPartialStride * 4));
+    if (matrix) {
+        splits = attention_chunk_splits(position, count, ws.limit > fixed ? ws.limit - fixed : 0);
+    }
+    const size_t partials = matrix && splits == 1 ? 0 : size_t(count) * kQueryHeads * splits * kPartialStride;
+    ws.ensure(fixed + Workspace::round(partials * 4));
     float *query_gate = ws.take<float>(size_t(count) * kQueryHeads * kQueryStride);
     float *attended = ws.take<float>(size_t(count) * kQueryHeads * kHeadSize);
-    float *partial = ws.take<float>(size_t(count) * kQueryHeads * splits * kPartialStride);
+    float *partial = ws.take<float>(partials);
     float *key = keys + static_cast<size_t>(position) * kKvHeads * kHeadSize;
     float *value = values + static_cast<size_t>(position) * kKvHeads * kHeadSize;
     project_qkv(ctx, L, inputs, count, query_gate, key, value, norm_in);
@@ -1237,12 +1205,18 @@ void full_attention_chunk(adi_hip_context *ctx, const adi_hip_full_attention *L,
            dim3(kHeadSize), 0, query_gate, key, L->query_norm, L->key_norm,
            count == 1 ? rope_table(position) : RopeTable{},
            count == 1 ? nullptr : rope_rows(ctx, position + count), position);
-    launch(ctx, "attention_partial", k_attention_partial, dim3(partial_blocks(splits), 1, count),
-           dim3(256), 0, static_cast<const float *>(query_gate), static_cast<const float *>(keys),
-           static_cast<const float *>(values), position, chunk, splits, partial);
-    launch(ctx, "attention_combine", k_attention_combine, dim3(kQueryHeads, count),
-           dim3(kHeadSize), 0, static_cast<const float *>(partial), splits,
-           static_cast<const float *>(query_gate), attended);
+    if (matrix) {
+        launch_attention_chunk(ctx, query_gate, keys, values, position, count, splits, partial, attended);
+    } else {
+        launch(ctx, "attention_partial", k_attention_partial, dim3(partial_blocks(splits), 1, count),
+               dim3(256), 0, static_cast<const float *>(query_gate), static_cast<const float *>(keys),
+               static_cast<const float *>(values), position, chunk, splits, partial);
+    }
+    if (!matrix || splits > 1) {
+        launch(ctx, "attention_combine", k_attention_combine, dim3(kQueryHeads, count),
+               dim3(kHeadSize), 0, static_cast<const float *>(partial), splits,
+               static_cast<const float *>(query_gate), attended);
+    }
     project_output(ctx, &L->output, attended, count, outputs, norm_tail);
 }
 

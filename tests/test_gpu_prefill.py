@@ -56,6 +56,71 @@ def test_full_attention_prefill(gpu, oracle, tluts):
         close(dv.cpu().numpy()[:end], values[:end], "values")
 
 
+@pytest.mark.parametrize("position,count", [(1016, 16), (1000, 17), (500, 47), (0, 256), (130, 129), (4000, 20)])
+def test_attention_chunk_edges(gpu, oracle, tluts, position, count):
+    """The matrix-core attention of a chunk at the edges of its 16-token
+    blocks and 32-key tiles, with one and several splits, against the oracle's
+    one-token form for the first, last and middle tokens (the caches as the
+    chunk left them). Scores and weights carry a float's relative error
+    (2^-22 at most per product), so outputs agree to the float noise of 32-bit
+    sums of up to 4020 terms: 1e-4 of the largest covers 4020 * 2^-24 = 2.4e-4
+    at a quarter of its worst case, as in the one-token tests."""
+    rng = syn.rng_for(66, position + count)
+    layer = syn.full_attention(rng, HIDDEN, tluts[1])
+    d = hip.upload_full_attention(gpu, layer, gpu.ne_codebook(tluts[1]))
+    held = po.FullAttentionStruct(layer)
+    capacity = position + count
+    dk = dev(rng.normal(0.0, 1.0, (capacity, 2, 256)).astype(np.float32))
+    dv = dev(rng.normal(0.0, 1.0, (capacity, 2, 256)).astype(np.float32))
+    x = syn.rms_normalized(syn.hidden_states(rng, count, HIDDEN))
+    out = torch.empty((count, HIDDEN), dtype=torch.float32, device="cuda")
+    hip.full_attention_prefill(gpu, d, position, count, dev(x), out, dk, dv, capacity)
+    keys, values = dk.cpu().numpy(), dv.cpu().numpy()
+    for b in sorted({0, 1, 15, count // 2, count - 1}):
+        want = po.full_attention_forward(oracle, held, position + b, x[b], keys.copy(), values.copy())
+        assert max_rel_error(out[b].cpu().numpy(), want) <= 1e-4, b
+
+
+@pytest.mark.parametrize("case", ["token", "key", "value", "large"])
+def test_attention_chunk_odd_values(gpu, tluts, case):
+    """Values the matrix cores' pieces cannot stand for: a NaN token (its row
+    and those after it are NaN, those before it are not), an infinity in the
+    history's keys or values, and finite values beyond f16 and bf16 give what
+    the vector kernel (chunks of 8 tokens) gives."""
+    rng = syn.rng_for(67, len(case))
+    layer = syn.full_attention(rng, HIDDEN, tluts[1])
+    d = hip.upload_full_attention(gpu, layer, gpu.ne_codebook(tluts[1]))
+    position, count = 600, 40
+    keys = rng.normal(0.0, 1.0, (position + count, 2, 256)).astype(np.float32)
+    values = rng.normal(0.0, 1.0, (position + count, 2, 256)).astype(np.float32)
+    x = syn.rms_normalized(syn.hidden_states(rng, count, HIDDEN))
+    if case == "token":
+        x[21, 5] = np.nan
+    elif case == "key":
+        keys[70, 0, 9] = np.inf
+    elif case == "value":
+        values[333, 1, 200] = -np.inf
+    else:
+        keys[70, 0, 9] = 3e5
+        values[599, 1, 3] = 3.4e38
+
+    def run(step):
+        dk, dv = dev(keys), dev(values)
+        out = torch.empty((count, HIDDEN), dtype=torch.float32, device="cuda")
+        for b in range(0, count, step):
+            hip.full_attention_prefill(gpu, d, position + b, step, dev(x[b:b + step]), out[b:b + step], dk, dv,
+                                       position + count)
+        return out.cpu().numpy()
+
+    got, want = run(count), run(8)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    if case == "token":
+        assert np.isfinite(got[:21]).all() and np.isnan(got[21:]).all()
+    for a, b in zip(got, want):
+        if np.isfinite(b).all():
+            assert max_rel_error(a, b) <= 1e-4
+
+
 def test_linear_attention_prefill(gpu, oracle, tluts):
     rng = syn.rng_for(62, 0)
     layer = syn.linear_attention(rng, HIDDEN, tluts[1])

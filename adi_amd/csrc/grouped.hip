@@ -97,15 +97,38 @@ struct ExpertWords {
     uint2 w[kFragments];
 };
 
+// The byte selectors of a lane's 28-bit string (its states 2 trow and 2 trow +
+// 1) in its two dwords, and of row 15's last byte in the tile's first dword.
+struct ExpertString {
+    uint32_t bytes, last;
+};
+
+// The selectors of tile row trow: its string starts at bit 24 trow of the
+// tile's stream, a whole byte, so one v_perm_b32 takes its four bytes from two
+// dwords (u16 words most significant byte first) and puts them in order. Row
+// 15's string ends in the tile's first byte (src/expert_trellis.hpp:79-80).
+__device__ __forceinline__ ExpertString expert_string(uint32_t trow) {
+    constexpr uint32_t kOrder = 0x67452301u;  // nibble j: where stream byte j of the two dwords lies
+    const uint32_t k = trow == 15u ? 5u : 3u * trow & 3u;
+    ExpertString out{0u, trow == 15u ? 0x07060501u : 0x07060504u};
+    for (uint32_t j = 0; j < 4u; ++j) {
+        out.bytes = out.bytes << 8 | (k + j < 8u ? kOrder >> 4u * (k + j) & 15u : 0x0Cu);
+    }
+    return out;
+}
+
+// The first of the two dwords a lane of tile row trow loads (row 15: 10, with
+// 11; its last byte comes from lane 0 of its row).
+__device__ __forceinline__ uint32_t expert_dwords(uint32_t trow) { return trow == 15u ? 10u : (24u * trow) >> 5; }
+
 // Everything about a wave's share of an item that does not change along K:
 // per-lane byte offsets (a K step advances the scalar offset only), the
-// lane's window shifts and its gamma row in LDS.
+// lane's byte selectors and its gamma row in LDS.
 struct ExpertWave {
     __amdgpu_buffer_rsrc_t words;
     uint32_t woff[kFragments];  // the lane's stream dword pair of fragment f at K step 0
     const uint2 *gammas;        // gamma row tsub + kh of the item, at the wave's first tile row
-    uint32_t sh0, sh1;          // shifts of the lane's two windows in the 64-bit string
-    bool row15;                 // the lane holds tile row 15, whose last window wraps
+    ExpertString string;
 };
 
 __device__ __forceinline__ void expert_words(const ExpertWave &wv, uint32_t kc, ExpertWords &s) {
@@ -122,11 +145,47 @@ struct ExpertA {
     half8 hi[kFragments], lo[kFragments];
 };
 
+// The lane's two half-states of a tile row: their hashes (bit 15 negates
+// component 0) and codebook entries.
+struct ExpertEntries {
+    uint32_t p0, p1;
+    uint2 e0, e1;
+};
+
+__device__ __forceinline__ ExpertEntries expert_gather(ExpertString at, uint2 words, const uint2 *plane) {
+    // row 15's last byte is in dword 0 of its tile, which lane 0 of the same
+    // 16-lane row (the same tile) loaded first (row_ror:15 reads lane (i + 1)
+    // mod 16)
+    const uint32_t wrap = __builtin_amdgcn_update_dpp(0u, words.x, 0x12F, 0xF, 0xF, false);
+    const uint32_t most = __builtin_amdgcn_perm(words.y, words.x, at.bytes);
+    const uint32_t string = __builtin_amdgcn_perm(most, wrap, at.last);
+    ExpertEntries out;
+    out.p0 = state_hash_low16(string >> 16);
+    out.p1 = state_hash_low16(string >> 4);
+    out.e0 = plane[(out.p0 >> 1) & 0x3FFFu];
+    out.e1 = plane[(out.p1 >> 1) & 0x3FFFu];
+    return out;
+}
+
+// The lane's eight values times the tile's gamma, as hi + lo.
+template <int PASSES>
+__device__ __forceinline__ void expert_scale(const ExpertEntries &in, uint32_t gamma, uint32_t sign_mask, half8 &hi,
+                                             half8 &lo) {
+#pragma clang fp contract(off)
+    const half8 v = __builtin_bit_cast(half8, u32x4{in.e0.x ^ (in.p0 & sign_mask), in.e0.y,
+                                                    in.e1.x ^ (in.p1 & sign_mask), in.e1.y});
+    const _Float16 g = __builtin_bit_cast(_Float16, static_cast<uint16_t>(gamma));
+    const half8 gv = {g, g, g, g, g, g, g, g};
+    hi = gv * v;
+    if constexpr (PASSES == 3) {
+        lo = __builtin_elementwise_fma(gv, v, -hi);
+    }
+}
+
 // Decodes the lane's A fragments at K step kc (lo only when PASSES is 3).
 template <int PASSES>
 __device__ __forceinline__ void expert_decode(const ExpertWave &wv, uint32_t kc, uint32_t sign_mask,
                                               const uint2 *plane, const ExpertWords &s, ExpertA &a) {
-#pragma clang fp contract(off)
     // gammas of the lane's tiles: fragment (rb, c) sits 2 rb + 2 c anti-diagonals
     // past the lane's first, so offsets 0, 2, 2, 4 of the lane's gamma row
     const uint2 g03 = wv.gammas[kc];
@@ -134,28 +193,7 @@ __device__ __forceinline__ void expert_decode(const ExpertWave &wv, uint32_t kc,
     const uint32_t gbits[kFragments] = {g03.x & 0xFFFFu, g03.y & 0xFFFFu, g03.y & 0xFFFFu, g47.x & 0xFFFFu};
 #pragma unroll
     for (int f = 0; f < kFragments; ++f) {
-        // row 15's second dword is dword 0 of its tile, which lane 0 of the
-        // same 16-lane row (the same tile) loaded first (row_ror:15 reads
-        // lane (i + 1) mod 16)
-        const uint32_t wrap = __builtin_amdgcn_update_dpp(0u, s.w[f].x, 0x12F, 0xF, 0xF, false);
-        const uint32_t d0 = wv.row15 ? s.w[f].y : s.w[f].x;
-        const uint32_t d1 = wv.row15 ? wrap : s.w[f].y;
-        // the lane's four stream words, most significant bit first
-        const uint64_t bits = (static_cast<uint64_t>(__builtin_amdgcn_alignbit(d0, d0, 16)) << 32) |
-                              __builtin_amdgcn_alignbit(d1, d1, 16);
-        const uint32_t p0 = state_hash_low16(static_cast<uint32_t>(bits >> wv.sh0));
-        const uint32_t p1 = state_hash_low16(static_cast<uint32_t>(bits >> wv.sh1));
-        uint2 e0 = plane[(p0 >> 1) & 0x3FFFu];
-        uint2 e1 = plane[(p1 >> 1) & 0x3FFFu];
-        e0.x ^= p0 & sign_mask;
-        e1.x ^= p1 & sign_mask;
-        const half8 v = __builtin_bit_cast(half8, u32x4{e0.x, e0.y, e1.x, e1.y});
-        const _Float16 g = __builtin_bit_cast(_Float16, static_cast<uint16_t>(gbits[f]));
-        const half8 gv = {g, g, g, g, g, g, g, g};
-        a.hi[f] = gv * v;
-        if constexpr (PASSES == 3) {
-            a.lo[f] = __builtin_elementwise_fma(gv, v, -a.hi[f]);
-        }
+        expert_scale<PASSES>(expert_gather(wv.string, s.w[f], plane), gbits[f], sign_mask, a.hi[f], a.lo[f]);
     }
 }
 
@@ -201,6 +239,220 @@ __device__ __forceinline__ void expert_multiply(const ExpertA &a, const half8 (&
     }
 }
 
+// ---- slots of at most 16 positions -------------------------------------------
+//
+// Most slots of a decode batch or of a default prefill micro-batch hold one to
+// eight positions, where an item's time is its decode and the latency of each
+// K step. Here a unit is one slot times four tile rows of one entry, run by
+// one wave on its own with v_mfma_f32_16x16x32_f16 (sixteen columns, half the
+// matrix time of the 32-column form): no block barrier, so the waves of a SIMD
+// fill each other's waits, and the last units spread one to a CU. Lane l holds
+// row l % 16 of a tile row and, at K step kc, tile column 4 kc + l / 16. A
+// wave reads its x_hat columns from memory itself (2 KB a K step), loads four
+// K steps ahead straight across units, and gathers the codebook entries of the
+// next K step before it multiplies this one's. Both launches of a layer of 256
+// experts: 45 tokens (1.8 positions a slot) 154 -> 108 us, 128 tokens with
+// uniform routes (4 a slot) 204 -> 142, 128 with skewed ones 81 -> 77; what
+// bounds it now is vector issue, about 100 instructions a K step and wave.
+// Slots of 17 positions or more fill a 32-column item's matrix time and share
+// its x_hat, so they stay block items.
+
+constexpr uint32_t kSmallPositions = 16;
+constexpr uint32_t kSmallTileColumns = 128;  // the widest matrix whose gamma rows fit the ring's LDS
+// a unit's gamma rows, twice: entry i of row q is the gamma at anti-diagonal
+// i + q past the unit's first tile row
+constexpr uint32_t kSmallGammaRow = kSmallTileColumns / 4u + 1u;  // uint2 of four halves
+constexpr uint32_t kSmallGammas = 2u * 4u * kSmallGammaRow;       // uint2 per wave
+
+__host__ __device__ inline bool small_slots_supported(uint32_t tile_columns) {
+    return tile_columns >= 16u && tile_columns <= kSmallTileColumns;  // whole groups of four K steps
+}
+
+struct SmallUnit {
+    __amdgpu_buffer_rsrc_t words, x_hi, x_lo, gamma;
+    float *z;            // of the unit's first position
+    uint32_t x_off;      // the lane's x_hat row and K offset
+    uint32_t tile_row;   // the unit's first
+    uint32_t positions;
+};
+
+template <int PASSES>
+__device__ __forceinline__ void expert_small_slots(const ExpertMfmaJobs &J, uint32_t half, uint32_t first_unit,
+                                                   uint32_t second_unit, uint32_t stride, const uint2 *plane,
+                                                   const uint16_t *slots, uint32_t slot_count, uint2 *gammas) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t column = lane & 15u, kq = lane >> 4;
+    const uint32_t rows = J.expert[0].rows, tile_rows = J.expert[0].tile_rows, tc_shift = J.expert[0].tc_shift;
+    const uint32_t tile_columns = 1u << tc_shift, steps = tile_columns / 4u;
+    const uint32_t parts = (tile_rows + 3u) / 4u;
+    const uint32_t units = slot_count * J.expert_count * parts;
+    const uint32_t sign_mask = half == 0 ? 0x8000u : 0u;
+    const ExpertString string = expert_string(column);
+    const uint32_t lane_words = (kq * 12u + expert_dwords(column)) * 4u;
+    if (first_unit >= units) {
+        return;
+    }
+    const auto open = [&](uint32_t unit) {
+        const uint32_t part = unit % parts, entry = unit / parts;
+        const ExpertMfma &a = J.expert[entry % J.expert_count];
+        const uint32_t slot = __builtin_amdgcn_readfirstlane(slots[entry / J.expert_count]);
+        const uint4 info = J.slot_info != nullptr ? J.slot_info[slot] : make_uint4(0u, 0u, J.max_positions, 0u);
+        const uint32_t mat = __builtin_amdgcn_readfirstlane(info.x);
+        const uint32_t first = __builtin_amdgcn_readfirstlane(info.y);
+        const uint32_t positions = __builtin_amdgcn_readfirstlane(info.z) - first;
+        const uint32_t half_columns = a.columns >> 1;
+        const size_t plane_elems = static_cast<size_t>(a.positions) * half_columns;
+        SmallUnit out;
+        out.words = buffer_over(a.trellis + mat * a.trellis_stride, (tile_rows << tc_shift) * 48u);
+        out.x_hi = buffer_over(a.x_hi + half * plane_elems, static_cast<uint32_t>(plane_elems * 2u));
+        out.x_lo = buffer_over(a.x_lo + half * plane_elems, static_cast<uint32_t>(plane_elems * 2u));
+        out.gamma = buffer_over(a.gamma + mat * a.gamma_stride, (tile_rows + tile_columns) * 2u);
+        out.z = a.z + half * a.z_split_stride + static_cast<size_t>(first) * rows;
+        // columns past the slot repeat its last position and are never stored
+        out.x_off = ((first + min(column, positions - 1u)) * half_columns + 8u * kq) * 2u;
+        out.tile_row = 4u * part;
+        out.positions = positions;
+        return out;
+    };
+    // the gamma of anti-diagonal tile_row + e in slot R_t + C_t - 1 - d, one
+    // less past the main anti-diagonal (src/codec_cache.cpp:117-147); past the
+    // matrix 0, for tiles that are never stored
+    const auto load_gamma = [&](const SmallUnit &u, uint32_t e) {
+        const uint32_t d = u.tile_row + e;
+        const uint32_t slot = tile_rows + tile_columns - 1u - d - (d >= tile_columns ? 1u : 0u);
+        return static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(u.gamma, slot * 2u, 0, 0));
+    };
+    const auto store_gamma = [&](uint2 *to, uint32_t e, uint32_t g) {
+        uint16_t *row = reinterpret_cast<uint16_t *>(to);
+#pragma unroll
+        for (uint32_t q = 0; q < 4u; ++q) {
+            if (e - q < 4u * kSmallGammaRow) {  // e < q wraps: out of range
+                row[q * 4u * kSmallGammaRow + e - q] = static_cast<uint16_t>(g);
+            }
+        }
+    };
+    struct Step {
+        ExpertWords words;
+        half8 hi, lo;
+    };
+    const auto load_step = [&](const SmallUnit &u, uint32_t kc, Step &to) {
+#pragma unroll
+        for (uint32_t f = 0; f < kFragments; ++f) {
+            const uint32_t tr = min(u.tile_row + f, tile_rows - 1u);
+            to.words.w[f] = __builtin_bit_cast(
+                uint2, __builtin_amdgcn_raw_buffer_load_b64(u.words, lane_words, ((tr << tc_shift) + 4u * kc) * 48u, 0));
+        }
+        to.hi = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(u.x_hi, u.x_off, kc * 64u, 0));
+        to.lo = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(u.x_lo, u.x_off, kc * 64u, 0));
+    };
+    struct Gathered {
+        ExpertEntries f[kFragments];
+    };
+    const auto gather = [&](const ExpertWords &w) {
+        Gathered out;
+#pragma unroll
+        for (uint32_t f = 0; f < kFragments; ++f) {
+            out.f[f] = expert_gather(string, w.w[f], plane);
+        }
+        return out;
+    };
+
+    uint32_t next_unit = second_unit;
+    SmallUnit load = open(first_unit);
+    uint32_t g0 = load_gamma(load, lane), g1 = load_gamma(load, lane + 64u), g2 = load_gamma(load, lane + 128u);
+    Step ring[4];
+#pragma unroll
+    for (uint32_t s = 0; s < 4u; ++s) {
+        load_step(load, s, ring[s]);
+    }
+    uint32_t load_kc = 4u;
+    uint2 *gamma_now = gammas, *gamma_next = gammas + 4u * kSmallGammaRow;
+    store_gamma(gamma_now, lane, g0);
+    store_gamma(gamma_now, lane + 64u, g1);
+    store_gamma(gamma_now, lane + 128u, g2);
+    SmallUnit now = load;
+    bool more = false;  // `load` is past `now`
+    uint32_t kc = 0;
+    f32x4 acc[kFragments];
+#pragma unroll
+    for (uint32_t f = 0; f < kFragments; ++f) {
+        acc[f] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    Gathered entries = gather(ring[0].words);
+    for (;;) {
+        if (load_kc == steps) {
+            more = next_unit < units;
+            if (more) {
+                load = open(next_unit);
+                next_unit += stride;
+                g0 = load_gamma(load, lane);
+                g1 = load_gamma(load, lane + 64u);
+                g2 = load_gamma(load, lane + 128u);
+                load_kc = 0;
+            } else {
+                load_kc = steps - 4u;  // the last group again, unused
+            }
+        }
+#pragma unroll
+        for (uint32_t s = 0; s < 4u; ++s) {
+            const Gathered next = gather(ring[(s + 1u) & 3u].words);
+            const uint2 g = gamma_now[kq * kSmallGammaRow + kc + s];
+            __builtin_amdgcn_sched_barrier(0);
+            const uint32_t gamma[kFragments] = {g.x & 0xFFFFu, g.x >> 16, g.y & 0xFFFFu, g.y >> 16};
+            half8 hi[kFragments], lo[kFragments];
+#pragma unroll
+            for (uint32_t f = 0; f < kFragments; ++f) {
+                expert_scale<PASSES>(entries.f[f], gamma[f], sign_mask, hi[f], lo[f]);
+            }
+#pragma unroll
+            for (uint32_t f = 0; f < kFragments; ++f) {
+                acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[f], ring[s].hi, acc[f], 0, 0, 0);
+            }
+#pragma unroll
+            for (uint32_t f = 0; f < kFragments; ++f) {
+                acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[f], ring[s].lo, acc[f], 0, 0, 0);
+            }
+            if constexpr (PASSES == 3) {
+#pragma unroll
+                for (uint32_t f = 0; f < kFragments; ++f) {
+                    acc[f] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[f], ring[s].hi, acc[f], 0, 0, 0);
+                }
+            }
+            load_step(load, load_kc + s, ring[s]);
+            entries = next;
+        }
+        load_kc += 4u;
+        kc += 4u;
+        if (kc == steps) {
+            // D register r of lane l: position l % 16, tile row's row 4 (l / 16) + r
+            if (column < now.positions) {
+#pragma unroll
+                for (uint32_t f = 0; f < kFragments; ++f) {
+                    if (now.tile_row + f < tile_rows) {
+                        *reinterpret_cast<f32x4 *>(now.z + static_cast<size_t>(column) * rows +
+                                                   (now.tile_row + f) * kTile + 4u * kq) = acc[f];
+                    }
+                }
+            }
+            if (!more) {
+                return;
+            }
+            uint2 *const spent = gamma_now;
+            gamma_now = gamma_next;
+            gamma_next = spent;
+            store_gamma(gamma_now, lane, g0);
+            store_gamma(gamma_now, lane + 64u, g1);
+            store_gamma(gamma_now, lane + 128u, g2);
+            now = load;
+            kc = 0;
+#pragma unroll
+            for (uint32_t f = 0; f < kFragments; ++f) {
+                acc[f] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+    }
+}
+
 // Block b serves codebook plane (b / 8) % 2 as worker ((b / 16) * 8 + b % 8)
 // (the two blocks that walk the same tiles share an XCD). Each block counts
 // the items of every routed slot (position groups x row quarters) and scans
@@ -227,12 +479,15 @@ __global__ __launch_bounds__(512 * GROUPS) void k_expert_mfma(ExpertMfmaJobs J) 
     // constant, so a gather's address is the masked row offset alone
     __shared__ uint4 plane_lds[kPlaneRows16];
     __shared__ uint32_t starts[kSlotCapacity + 1];
-    __shared__ uint32_t wave_sums[kWaves];
+    __shared__ uint64_t wave_sums[kWaves];
+    __shared__ uint32_t small_count;
     // gamma rows of an item: row q entry i = gamma of the tile at
     // anti-diagonal tr_block + i + q; lane (w, tsub, kh) reads its tiles'
     // gammas at K step kc from row tsub + kh at entries 4w + 4kc .. + 7
     __shared__ uint2 gamma_rows[kExpertGroups][4][kGammaRow / 4];
     __shared__ uint4 b_ring[kExpertGroups][2][kBSlot / 16];
+    static_assert(sizeof(b_ring) >= 8u * kExpertGroups * kSmallGammas * sizeof(uint2), "the waves' gamma rows");
+    __shared__ uint16_t small_slots[kSlotCapacity];
     const uint32_t b = blockIdx.x;
     const uint32_t half = (b >> 3) & 1u;
     const uint32_t worker = ((b >> 4) << 3) | (b & 7u);
@@ -251,9 +506,11 @@ __global__ __launch_bounds__(512 * GROUPS) void k_expert_mfma(ExpertMfmaJobs J) 
         for (uint32_t u = 0; u < kPer; ++u) {
             v[u] = src[min(u * kExpertThreads + threadIdx.x, kPlaneRows16 - 1u)];
         }
-        // item counts per slot: each thread owns two consecutive slots
+        // item counts per slot: each thread owns two consecutive slots; a
+        // small slot counts 1 in the upper half instead
         const uint32_t quarters = J.row_groups;
         uint32_t count[2];
+        bool small[2];
 #pragma unroll
         for (uint32_t k = 0; k < 2; ++k) {
             const uint32_t s = 2u * threadIdx.x + k;
@@ -262,14 +519,17 @@ __global__ __launch_bounds__(512 * GROUPS) void k_expert_mfma(ExpertMfmaJobs J) 
                 info = J.slot_info != nullptr ? J.slot_info[s]
                                               : make_uint4(0u, 0u, s == 0 ? J.max_positions : 0u, 0u);
             }
-            count[k] = info.z > info.y ? (info.z - info.y + kPositions - 1u) / kPositions * quarters : 0u;
+            const uint32_t held = info.z > info.y ? info.z - info.y : 0u;
+            small[k] = J.small_slots != 0u && held != 0u && held <= kSmallPositions;
+            count[k] = small[k] ? 0u : (held + kPositions - 1u) / kPositions * quarters;
         }
-        // block-wide exclusive scan of the counts (slot order)
-        const uint32_t own = count[0] + count[1];
-        uint32_t inclusive = own;
+        // block-wide exclusive scans (slot order): items in the lower half,
+        // small slots in the upper
+        const uint64_t own = (static_cast<uint64_t>(small[0]) + small[1]) << 32 | (count[0] + count[1]);
+        uint64_t inclusive = own;
 #pragma unroll
         for (int offset = 1; offset < 64; offset <<= 1) {
-            const uint32_t other = static_cast<uint32_t>(__shfl_up(static_cast<int>(inclusive), offset));
+            const uint64_t other = __shfl_up(static_cast<unsigned long long>(inclusive), offset);
             if (lane >= static_cast<uint32_t>(offset)) {
                 inclusive += other;
             }
@@ -282,17 +542,27 @@ __global__ __launch_bounds__(512 * GROUPS) void k_expert_mfma(ExpertMfmaJobs J) 
             plane_lds[min(u * kExpertThreads + threadIdx.x, kPlaneRows16 - 1u)] = v[u];
         }
         __syncthreads();
-        uint32_t before = 0;
+        uint64_t before = 0;
         for (uint32_t w = 0; w < wave; ++w) {
             before += wave_sums[w];
         }
-        const uint32_t exclusive = before + inclusive - own;
+        const uint64_t exclusive = before + inclusive - own;
         if (2u * threadIdx.x < kSlotCapacity) {
-            starts[2u * threadIdx.x] = exclusive;
-            starts[2u * threadIdx.x + 1u] = exclusive + count[0];
+            const uint32_t start = static_cast<uint32_t>(exclusive);
+            starts[2u * threadIdx.x] = start;
+            starts[2u * threadIdx.x + 1u] = start + count[0];
+            uint32_t place = static_cast<uint32_t>(exclusive >> 32);
+#pragma unroll
+            for (uint32_t k = 0; k < 2; ++k) {
+                if (small[k]) {
+                    small_slots[place] = static_cast<uint16_t>(2u * threadIdx.x + k);
+                    ++place;
+                }
+            }
         }
         if (threadIdx.x == kExpertThreads - 1u) {
-            starts[kSlotCapacity] = before + inclusive;  // items per entry
+            starts[kSlotCapacity] = static_cast<uint32_t>(before + inclusive);  // items per entry
+            small_count = static_cast<uint32_t>((before + inclusive) >> 32);
         }
     }
     __syncthreads();
@@ -302,6 +572,7 @@ __global__ __launch_bounds__(512 * GROUPS) void k_expert_mfma(ExpertMfmaJobs J) 
     const uint32_t m = lane & 31u, kh = lane >> 5;   // MFMA row / column and K half
     const uint32_t trow = m & 15u, tsub = m >> 4;    // row within the tile, tile row within the block
     const uint32_t sign_mask = half == 0 ? 0x8000u : 0u;
+    const ExpertString string = expert_string(trow);
     // the thread's share of its group's B loads: one chunk of one B row (B
     // rows are (hi/lo, position); wave w of the group loads rows
     // (64 / kThreadsPerRow) w .., so the hi/lo plane is wave-uniform: derived
@@ -363,13 +634,7 @@ __global__ __launch_bounds__(512 * GROUPS) void k_expert_mfma(ExpertMfmaJobs J) 
         ExpertWave wv;
         const uint32_t tiles = a.tile_rows << a.tc_shift;
         wv.words = buffer_over(a.trellis + mat * a.trellis_stride, tiles * 48u);
-        // the lane's states 2 trow, 2 trow + 1 start in dword dw = 24 trow / 32;
-        // row 15's second window wraps to dword 0 of its tile
-        // (src/expert_trellis.hpp:79-80), so that lane loads dwords 10 and 11
-        // and takes dword 0 from lane 0 of its 16-lane row
-        const uint32_t dw = (24u * trow) >> 5;
-        wv.row15 = trow == 15u;
-        const uint32_t dpair = wv.row15 ? 10u : dw;
+        const uint32_t dpair = expert_dwords(trow);
 #pragma unroll
         for (int f = 0; f < kFragments; ++f) {
             const uint32_t rb = f >> 1, c = f & 1;
@@ -378,9 +643,7 @@ __global__ __launch_bounds__(512 * GROUPS) void k_expert_mfma(ExpertMfmaJobs J) 
             wv.woff[f] = (tile * 12u + dpair) * 4u;
         }
         wv.gammas = gamma_rows[group][tsub + kh] + gwave;  // entry 4 * gwave
-        const uint32_t pos = (24u * trow) & 31u;  // bit of state 2 trow in dword dw
-        wv.sh0 = 48u - pos;
-        wv.sh1 = 36u - pos;
+        wv.string = string;
 
         // the previous item's readers of the gamma rows and the ring are done
         __syncthreads();
@@ -520,6 +783,20 @@ __global__ __launch_bounds__(512 * GROUPS) void k_expert_mfma(ExpertMfmaJobs J) 
                 }
             }
         }
+    }
+    // the small slots, a unit a wave: first the workers that the last round of
+    // items left idle take one a wave, then all take the rest in turn, worker
+    // by worker, so that the last ones spread over the CUs
+    if (small_count != 0u) {  // uniform over the block
+        __syncthreads();      // the ring is free
+        const uint32_t busy = rounds % workers, idle = busy == 0u ? 0u : workers - busy;
+        const uint32_t stride = workers * kWaves;
+        const uint32_t turn = idle * kWaves + worker + workers * wave;
+        const bool extra = idle != 0u && worker >= busy;
+        const uint32_t first_unit = extra ? worker - busy + idle * wave : turn;
+        expert_small_slots<PASSES>(J, half, first_unit, extra ? turn : turn + stride, stride, plane, small_slots,
+                                   small_count,
+                                   reinterpret_cast<uint2 *>(&b_ring[0][0][0]) + wave * kSmallGammas);
     }
 }
 
@@ -710,6 +987,7 @@ void launch_expert_mfma(adi_hip_context *ctx, ExpertMfmaJobs &J) {
     J.row_groups = ceil_div(e.rows / kTile, kBlockTileRows);  // row quarters of an item
     J.position_groups = ceil_div(J.max_positions, 32u * kExpertCB);
     J.items = J.expert_count * J.max_active * J.position_groups * J.row_groups;  // upper bound
+    J.small_slots = small_slots_supported(e.columns / kTile) ? 1u : 0u;
     const uint32_t cap = ctx->cu_count >= 16 ? ctx->cu_count / 16 * 16 : 16u;
     const uint32_t needed = 16u * ceil_div(ceil_div(J.items, kExpertGroups), 8u);
     const uint32_t blocks = needed < cap ? needed : cap;

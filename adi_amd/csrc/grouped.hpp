@@ -74,6 +74,7 @@ struct ExpertMfmaJobs {
     uint32_t row_groups;
     uint32_t position_groups;
     uint32_t items;            // per plane
+    uint32_t small_slots;      // whether slots of few positions run as units of a wave
 };
 
 struct NeMfmaJobs {

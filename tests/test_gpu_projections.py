@@ -71,6 +71,26 @@ def test_expert_matmul(gpu, books, oracle, rows, columns, batch):
 MFMA_TOL = 1e-4
 
 
+@pytest.mark.parametrize("rows,columns", [(16, 256), (32, 256), (128, 512), (512, 2048), (64, 4096)])
+@pytest.mark.parametrize("batch", [16, 17])
+def test_expert_slot_of_sixteen(gpu, books, oracle, rows, columns, batch):
+    """At 16 positions a slot runs as units of four tile rows a wave (fewer
+    tile rows than that, one group of K steps, the widest matrix but one), at
+    17 as a block's item, and 4096 columns always do. hi + lo hold 22 bits of
+    each factor and the left-out product is below 2^-22, so a sum of 4096
+    random-sign terms stays within 64 * 2^-22 = 1.5e-5 of a term, under 1e-6
+    of the largest output; 1e-5 leaves room for the float sums' order."""
+    et, _, eb, _ = books
+    rng = syn.rng_for(0, 9 * rows + columns + batch)
+    m = syn.expert_matrix(rng, rows, columns, et)
+    x = syn.hidden_states(rng, batch, columns)
+    want = po.expert_matmul(oracle, m, x)
+    dm = hip.upload_expert(gpu, m, eb)
+    out = torch.empty((batch, rows), dtype=torch.float32, device="cuda")
+    hip.expert_matmul(gpu, dm, gpu.to_device(x), batch, out)
+    assert max_rel_error(out.cpu().numpy(), want) <= 1e-5
+
+
 @pytest.mark.parametrize("rows,columns", [(16, 64), (64, 128), (512, 2048), (2048, 512)])
 @pytest.mark.parametrize("batch", [16, 33, 64, 100, 300])
 def test_expert_matmul_mfma(gpu, books, oracle, rows, columns, batch):

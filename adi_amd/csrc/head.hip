@@ -23,6 +23,7 @@
 #include "dense.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace adi_hip {
 namespace {
@@ -286,6 +287,41 @@ __device__ __forceinline__ hm_f32x4 hm_mfma(hm_u32x4 a, hm_u32x4 b, hm_f32x4 c) 
                                                     __builtin_bit_cast(hm_bf16x8, b), c, 0, 0, 0);
 }
 
+// One token's 16 columns at x (quarter q of a group), of MFMA i: the fragments
+// of its three pieces, and the partial sums of K of the pieces and of the
+// bound column (sum[3]).
+struct HeadFragments {
+    hm_u32x4 frag[3];
+    float sum[4];
+};
+__device__ __forceinline__ HeadFragments hm_fragments(const float *__restrict__ x, bool live, uint32_t i) {
+#pragma clang fp contract(off)
+    HeadFragments out{};
+    float bound = 0.0f;
+#pragma unroll
+    for (uint32_t d = 0; d < 4; ++d) {
+        uint32_t half[3][2];
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) {
+            const float xv = live ? x[hm_code(i, d, h)] : 0.0f;
+            const float v = xv * (h == 0 ? 32.0f : 64.0f);  // exact
+            const float f = h == 0 ? 1.5f : 1.25f;           // 1 + 16 delta
+#pragma unroll
+            for (uint32_t p = 0; p < 3; ++p) {
+                half[p][h] = hm_piece(v, p);
+                out.sum[p] += __uint_as_float(half[p][h] << 16) * f;
+            }
+            bound += fabsf(xv);
+        }
+#pragma unroll
+        for (uint32_t p = 0; p < 3; ++p) {
+            out.frag[p][d] = half[p][0] | (half[p][1] << 16);
+        }
+    }
+    out.sum[3] = -16.0f * bound;
+    return out;
+}
+
 // The B fragments and accumulator starts of tokens t0 .. t0 + 3 (zero past
 // `batch`) into LDS; ends with a block barrier.
 __device__ void hm_build_tables(HeadMfmaLds &L, const float *__restrict__ x, uint32_t t0,
@@ -299,35 +335,12 @@ __device__ void hm_build_tables(HeadMfmaLds &L, const float *__restrict__ x, uin
         const float *xt = x + static_cast<size_t>(live ? t0 + t : 0) * 2048u + 64u * g + 16u * q;
 #pragma unroll
         for (uint32_t i = 0; i < 2; ++i) {
-            hm_u32x4 frag[3];
-            float sum[3] = {0.0f, 0.0f, 0.0f}, bound = 0.0f;
+            const HeadFragments f = hm_fragments(xt, live, i);
 #pragma unroll
-            for (uint32_t d = 0; d < 4; ++d) {
-                uint32_t half[3][2];
-#pragma unroll
-                for (uint32_t h = 0; h < 2; ++h) {
-                    const float xv = live ? xt[hm_code(i, d, h)] : 0.0f;
-                    const float v = xv * (h == 0 ? 32.0f : 64.0f);  // exact
-                    const float f = h == 0 ? 1.5f : 1.25f;           // 1 + 16 delta
-#pragma unroll
-                    for (uint32_t p = 0; p < 3; ++p) {
-                        half[p][h] = hm_piece(v, p);
-                        sum[p] += __uint_as_float(half[p][h] << 16) * f;
-                    }
-                    bound += fabsf(xv);
-                }
-#pragma unroll
-                for (uint32_t p = 0; p < 3; ++p) {
-                    frag[p][d] = half[p][0] | (half[p][1] << 16);
-                }
+            for (uint32_t p = 0; p < 4; ++p) {
+                L.b[g][i][q][4 * t + p] = p < 3 ? f.frag[p] : hm_u32x4{0u, 0u, 0u, 0u};
+                L.u.part[g][4 * t + p][4 * i + q] = f.sum[p];
             }
-#pragma unroll
-            for (uint32_t p = 0; p < 3; ++p) {
-                L.b[g][i][q][4 * t + p] = frag[p];
-                L.u.part[g][4 * t + p][4 * i + q] = sum[p];
-            }
-            L.b[g][i][q][4 * t + 3] = hm_u32x4{0u, 0u, 0u, 0u};
-            L.u.part[g][4 * t + 3][4 * i + q] = -16.0f * bound;
         }
     }
     __syncthreads();
@@ -606,6 +619,285 @@ __global__ __launch_bounds__(kHmThreads) void k_head_mfma(
                 best.value[at] = best_v;
                 best.index[at] = best_i;
                 best.upper[at] = upper;
+            }
+        }
+    }
+}
+
+// ---- five to sixteen tokens in one pass over the codes ------------------------
+//
+// The arithmetic of k_head_mfma (the same bits) for up to sixteen tokens at
+// once. Their pieces are columns 3 t + p of up to three tables of sixteen
+// columns (no bound columns). The fragments of the whole width would not fit
+// the LDS, so a block keeps them for a quarter of the columns (8 groups) at a
+// time: quarter by quarter it builds the tables and runs its row tiles over
+// that quarter's codes, each tile's sums staying in registers. A wave runs two
+// tiles together, so that a fragment read from LDS feeds two products, and
+// reads the next step's fragments and codes from LDS under them. The codes are
+// read and decoded once for all tokens: 151,936 rows at 5, 8, 10 and 16 tokens
+// take 54, 67, 69 and 86 us, passes of four tokens 83, 83, 122 and 159. What
+// bounds it is vector issue (the decode, the scaled sums) at two waves a SIMD
+// and the waits at the four table builds. Up to four tokens k_head_mfma's one
+// pass takes 41.
+// A wave holds the sums of five tiles: two pairs, then a single tile (151,936
+// rows are 4.6 tiles a wave; three pairs left a third of the waves idle for
+// half of their time).
+constexpr uint32_t kHmRounds = 3;
+constexpr uint32_t kHmSetTiles = 5;
+__host__ __device__ constexpr uint32_t hm_tiles_of(uint32_t round) { return round < 2u ? 2u : 1u; }
+constexpr uint32_t kHmManyTokens = 16;
+
+template <uint32_t TABLES>
+struct HeadManyLds {
+    hm_u32x4 b[TABLES][kHmChunk][2][4][16];
+    float c[TABLES][kHmChunk][16];
+    uint16_t scale[kHmWaves][2][kHmChunk][kHmTile];
+    union {
+        float part[TABLES][kHmChunk][16][8];  // while the tables build
+        uint32_t stage[kHmWaves][2][kHmTile * kHmStagePitch / 4];
+        float sums[kHmWaves][kHmTile][16 * TABLES + 1];  // a tile's columns, at the end
+    } u;
+};
+
+// Tokens 0 .. batch - 1 (3 batch <= 16 TABLES) of x [batch][2048] into logits
+// [batch][rows]. The codes are 16-byte aligned.
+template <uint32_t TABLES>
+__global__ __launch_bounds__(kHmThreads) void k_head_mfma_many(const uint8_t *__restrict__ packed,
+                                                               const uint16_t *__restrict__ scales, uint32_t rows,
+                                                               const float *__restrict__ x, uint32_t batch,
+                                                               float *__restrict__ logits) {
+#pragma clang fp contract(off)
+    extern __shared__ __align__(16) unsigned char hm_raw[];
+    HeadManyLds<TABLES> &L = *reinterpret_cast<HeadManyLds<TABLES> *>(hm_raw);
+    const uint32_t lane = threadIdx.x & 63u;
+    // scalar, so that the tiles' loads take a constant lane offset and a scalar
+    // one
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
+    const uint32_t wave_global = blockIdx.x * kHmWaves + wave;
+    const uint32_t wave_count = gridDim.x * kHmWaves;
+    const uint32_t tiles = (rows + kHmTile - 1u) / kHmTile;
+    const uint32_t q = lane / 16u, n = lane % 16u;
+    const uint32_t shift = 16u * (q & 1u);
+    // loads past the last row give zeros
+    const __amdgpu_buffer_rsrc_t code_buffer =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(packed), 0, rows * 1280u, 0x00020000);
+    const __amdgpu_buffer_rsrc_t scale_buffer =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(scales), 0, rows * 64u, 0x00020000);
+    struct Raw {
+        hm_u32x4 codes[2][kHmRawLoads];
+        hm_u32x4 scales;
+    };
+    // piece e = 64 k + lane of a tile's quarter: row e / 20, bytes 16 (e % 20) ..
+    uint32_t code_from[kHmRawLoads], code_to[kHmRawLoads];
+#pragma unroll
+    for (uint32_t k = 0; k < kHmRawLoads; ++k) {
+        const uint32_t e = 64u * k + lane;
+        code_from[k] = e / 20u * 1280u + 16u * (e % 20u);
+        code_to[k] = (e / 20u * kHmStagePitch + 16u * (e % 20u)) / 4u;
+    }
+    const uint32_t scale_from = (lane & 31u) * 64u;
+    // quarter kq of the codes and scales (lanes 0-31: a row's 8 groups) of
+    // `count` tiles
+    const auto load = [&]<uint32_t COUNT>(std::integral_constant<uint32_t, COUNT>, uint32_t tile0, uint32_t kq,
+                                          Raw &out) {
+#pragma unroll
+        for (uint32_t tile = 0; tile < COUNT; ++tile) {
+            const uint32_t at = (tile0 + tile) * kHmTile * 1280u + kHmPieceBytes * kq;
+#pragma unroll
+            for (uint32_t k = 0; k < kHmRawLoads; ++k) {
+                out.codes[tile][k] = __builtin_bit_cast(
+                    hm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(code_buffer, code_from[k], at, 0));
+            }
+        }
+        out.scales = __builtin_bit_cast(hm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      scale_buffer, scale_from, tile0 * kHmTile * 64u + 16u * kq, 0));
+    };
+    using One = std::integral_constant<uint32_t, 1>;
+    using Two = std::integral_constant<uint32_t, 2>;
+    const auto fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    // the lane's staged codes and scales of group j of the round's tiles
+    struct GroupIn {
+        uint32_t w[2][3];
+        hm_u32x2 s[2];
+    };
+    const uint32_t *const codes_at = &L.u.stage[wave][0][(n * kHmStagePitch + 10u * q - 2u * (q & 1u)) / 4u];
+    const auto read_group = [&](uint32_t j, uint32_t held) {
+        GroupIn out{};
+#pragma unroll
+        for (uint32_t tile = 0; tile < held; ++tile) {
+#pragma unroll
+            for (uint32_t i = 0; i < 3; ++i) {
+                out.w[tile][i] = codes_at[tile * (kHmTile * kHmStagePitch / 4u) + 10u * j + i];
+            }
+            out.s[tile] = *reinterpret_cast<const hm_u32x2 *>(&L.scale[wave][tile][j][4u * q]);
+        }
+        return out;
+    };
+    struct TableIn {
+        hm_u32x4 b0, b1;
+        float c;
+    };
+    const auto read_table = [&](uint32_t j, uint32_t table) {
+        return TableIn{L.b[table][j][0][q][n], L.b[table][j][1][q][n], L.c[table][j][n]};
+    };
+
+    // every block runs the same number of rounds (its barriers)
+    for (uint32_t first = 0; first < tiles; first += kHmSetTiles * wave_count) {
+        // the wave's first tile of round r
+        const auto tile_of = [&](uint32_t r) {
+            return first + 2u * r * wave_count + hm_tiles_of(r) * wave_global;
+        };
+        hm_f32x4 out[kHmRounds][2][TABLES];
+#pragma unroll
+        for (uint32_t r = 0; r < kHmRounds; ++r) {
+#pragma unroll
+            for (uint32_t tile = 0; tile < 2; ++tile) {
+#pragma unroll
+                for (uint32_t table = 0; table < TABLES; ++table) {
+                    out[r][tile][table] = hm_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+            }
+        }
+        Raw raw;
+        load(Two{}, tile_of(0), 0, raw);
+        for (uint32_t kq = 0; kq < 4u; ++kq) {
+            __syncthreads();  // the previous quarter's readers are done
+            if (threadIdx.x < kHmChunk * 4u * kHmManyTokens) {
+                const uint32_t t = threadIdx.x % kHmManyTokens, rest = threadIdx.x / kHmManyTokens;
+                const uint32_t tq = rest % 4u, g = rest / 4u;
+                const bool live = t < batch;
+                const float *xt = x + static_cast<size_t>(live ? t : 0u) * 2048u + 64u * (kHmChunk * kq + g) + 16u * tq;
+#pragma unroll
+                for (uint32_t i = 0; i < 2; ++i) {
+                    const HeadFragments f = hm_fragments(xt, live, i);
+#pragma unroll
+                    for (uint32_t p = 0; p < 3; ++p) {
+                        const uint32_t column = 3u * t + p;
+                        if (column < 16u * TABLES) {
+                            L.b[column / 16u][g][i][tq][column % 16u] = f.frag[p];
+                            L.u.part[column / 16u][g][column % 16u][4u * i + tq] = f.sum[p];
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            // (the one column past 3 batch of a last table holds old values,
+            // or none yet; nothing reads its sums)
+            if (threadIdx.x < TABLES * kHmChunk * 16u) {
+                const float *part = &L.u.part[0][0][0][0] + 8u * threadIdx.x;
+                float k = 0.0f;
+#pragma unroll
+                for (uint32_t j = 0; j < 8; ++j) {
+                    k += part[j];
+                }
+                (&L.c[0][0][0])[threadIdx.x] = -k;
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t r = 0; r < kHmRounds; ++r) {
+                constexpr uint32_t kLast = kHmRounds - 1u;
+                const uint32_t held = hm_tiles_of(r);
+                if (tile_of(r) < tiles) {  // the same for the wave
+                    // the tiles' quarter into the wave's LDS, the registers
+                    // then reloaded with the wave's next quarter
+#pragma unroll
+                    for (uint32_t tile = 0; tile < held; ++tile) {
+#pragma unroll
+                        for (uint32_t k = 0; k < kHmRawLoads; ++k) {
+                            *reinterpret_cast<hm_u32x4 *>(&L.u.stage[wave][tile][code_to[k]]) = raw.codes[tile][k];
+                        }
+                    }
+                    if (lane < 32u) {
+#pragma unroll
+                        for (uint32_t e = 0; e < 8; ++e) {
+                            L.scale[wave][lane / 16u][e][lane % 16u] =
+                                static_cast<uint16_t>(raw.scales[e / 2] >> (16u * (e % 2u)));
+                        }
+                    }
+                    if (r == 0u || r == kLast || tile_of(r + 1u) >= tiles) {
+                        const bool next = r < kLast && tile_of(r + 1u) < tiles;
+                        load(Two{}, tile_of(next ? r + 1u : 0u), next ? kq : min(kq + 1u, 3u), raw);
+                    } else {
+                        load(One{}, tile_of(kLast), kq, raw);
+                    }
+                    fence();
+                    GroupIn in = read_group(0, held);
+                    TableIn b = read_table(0, 0);
+#pragma unroll
+                    for (uint32_t j = 0; j < kHmChunk; ++j) {
+                        hm_u32x4 a[2][2];
+                        hm_f32x4 s[2];
+#pragma unroll
+                        for (uint32_t tile = 0; tile < held; ++tile) {
+                            hm_decode(__builtin_amdgcn_alignbit(in.w[tile][1], in.w[tile][0], shift),
+                                      __builtin_amdgcn_alignbit(in.w[tile][2], in.w[tile][1], shift),
+                                      in.w[tile][2] >> shift, a[tile][0], a[tile][1]);
+                            const hm_u32x2 sb = in.s[tile];
+                            s[tile] = hm_f32x4{half_bits_to_float(sb.x & 0xFFFFu), half_bits_to_float(sb.x >> 16),
+                                               half_bits_to_float(sb.y & 0xFFFFu), half_bits_to_float(sb.y >> 16)};
+                        }
+                        in = read_group(min(j + 1u, kHmChunk - 1u), held);
+#pragma unroll
+                        for (uint32_t table = 0; table < TABLES; ++table) {
+                            const bool end = table + 1u == TABLES;
+                            const TableIn next = read_table(end ? min(j + 1u, kHmChunk - 1u) : j, end ? 0u : table + 1u);
+                            __builtin_amdgcn_sched_barrier(0);
+                            hm_f32x4 acc[2];
+#pragma unroll
+                            for (uint32_t tile = 0; tile < held; ++tile) {
+                                acc[tile] = hm_mfma(a[tile][0], b.b0, hm_f32x4{b.c, b.c, b.c, b.c});
+                            }
+#pragma unroll
+                            for (uint32_t tile = 0; tile < held; ++tile) {
+                                acc[tile] = hm_mfma(a[tile][1], b.b1, acc[tile]);
+                            }
+#pragma unroll
+                            for (uint32_t tile = 0; tile < held; ++tile) {
+                                hm_f32x4 &o = out[r][tile][table];
+                                o.x = fmaf(s[tile].x, acc[tile].x, o.x);
+                                o.y = fmaf(s[tile].y, acc[tile].y, o.y);
+                                o.z = fmaf(s[tile].z, acc[tile].z, o.z);
+                                o.w = fmaf(s[tile].w, acc[tile].w, o.w);
+                            }
+                            b = next;
+                        }
+                    }
+                    fence();  // every lane's reads end before the next tiles are staged
+                }
+            }
+        }
+        // the pieces of a token lie in three columns: through LDS, then lane l
+        // token l / 4, rows 4 (l % 4) .. + 3 of a tile
+        __syncthreads();  // the stages of all waves are free
+#pragma unroll
+        for (uint32_t r = 0; r < kHmRounds; ++r) {
+#pragma unroll
+            for (uint32_t tile = 0; tile < hm_tiles_of(r); ++tile) {
+#pragma unroll
+                for (uint32_t table = 0; table < TABLES; ++table) {
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        L.u.sums[wave][4u * q + j][16u * table + n] = out[r][tile][table][j];
+                    }
+                }
+                fence();
+                const uint32_t t = lane / 4u, row = 4u * (lane % 4u);
+                const uint32_t global = (tile_of(r) + tile) * kHmTile + row;
+                if (t < batch) {
+                    float *to = logits + static_cast<size_t>(t) * rows + global;
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        const float *piece = &L.u.sums[wave][row + j][3u * t];
+                        if (global + j < rows) {
+                            to[j] = (piece[0] + piece[1]) + piece[2];
+                        }
+                    }
+                }
+                fence();
             }
         }
     }
@@ -1019,6 +1311,27 @@ bool head_wave_best(const adi_hip_head_chunk *h) {
     return h->columns == 2048u && h->protected_count == 0;
 }
 
+// Logits of five to sixteen tokens (16-byte aligned codes).
+void launch_head_many(adi_hip_context *ctx, const adi_hip_head_chunk *h, const float *x, uint32_t batch,
+                      float *logits) {
+    const uint32_t pairs = ceil_div(ceil_div(h->rows, kHmTile), 2);
+    const dim3 blocks(std::min<uint32_t>(ceil_div(pairs, kHmWaves), static_cast<uint32_t>(ctx->cu_count)));
+    const auto run = [&](auto kernel, size_t lds) {
+        launch(ctx, "head_mfma", kernel, blocks, dim3(kHmThreads), lds, h->packed, h->group_scale_f16, h->rows, x,
+               batch, logits);
+    };
+    static const bool ready =
+        set_lds_limit(reinterpret_cast<const void *>(&k_head_mfma_many<1>), sizeof(HeadManyLds<1>)) &&
+        set_lds_limit(reinterpret_cast<const void *>(&k_head_mfma_many<2>), sizeof(HeadManyLds<2>)) &&
+        set_lds_limit(reinterpret_cast<const void *>(&k_head_mfma_many<3>), sizeof(HeadManyLds<3>));
+    (void)ready;
+    switch (ceil_div(3u * batch, 16)) {
+    case 1: return run(k_head_mfma_many<1>, sizeof(HeadManyLds<1>));
+    case 2: return run(k_head_mfma_many<2>, sizeof(HeadManyLds<2>));
+    default: return run(k_head_mfma_many<3>, sizeof(HeadManyLds<3>));
+    }
+}
+
 void head_logits(adi_hip_context *ctx, const adi_hip_head_chunk *h, const float *x,
                  uint32_t batch, float *logits, float *bounds,
                  HeadWaveBest best = HeadWaveBest{0.0f, nullptr, nullptr, nullptr}) {
@@ -1050,8 +1363,20 @@ void head_logits(adi_hip_context *ctx, const adi_hip_head_chunk *h, const float 
                 set_lds_limit(reinterpret_cast<const void *>(&k_head_mfma<true, false>), sizeof(HeadMfmaLds)) &&
                 set_lds_limit(reinterpret_cast<const void *>(&k_head_mfma<false, false>), sizeof(HeadMfmaLds));
             (void)ready;
-            launch(ctx, "head_mfma", kernel, dim3(wide), dim3(kHmThreads), sizeof(HeadMfmaLds),
-                   h->packed, h->group_scale_f16, h->rows, x, batch, logits, bounds, best);
+            // without bounds, five tokens and more go sixteen at a time through
+            // one pass over the codes, what is left (up to four) as before
+            uint32_t t0 = 0;
+            const bool addressed = size_t(h->rows) + 64u <= 0xFFFFFFFFu / 1280u;  // by 32-bit offsets
+            while (bounds == nullptr && coalesced && addressed && batch - t0 > kHmTokens) {
+                const uint32_t tokens = std::min(batch - t0, kHmManyTokens);
+                launch_head_many(ctx, h, x + size_t(t0) * 2048u, tokens, logits + size_t(t0) * h->rows);
+                t0 += tokens;
+            }
+            if (t0 < batch) {
+                launch(ctx, "head_mfma", kernel, dim3(wide), dim3(kHmThreads), sizeof(HeadMfmaLds),
+                       h->packed, h->group_scale_f16, h->rows, x + size_t(t0) * 2048u, batch - t0,
+                       logits + size_t(t0) * h->rows, bounds, best);
+            }
         } else if (batch == 1) {
             launch(ctx, "head_gemv", k_head_gemv<1>, dim3(blocks), dim3(256), 0, h->packed,
                    h->group_scale_f16, h->rows, h->columns, x, static_cast<const float *>(sums),

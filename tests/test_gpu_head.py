@@ -59,6 +59,25 @@ def test_head_2048_columns_by_batch(gpu, oracle, batch):
     assert np.array_equal(arg, np.argmax(want, axis=1).astype(np.uint32))
 
 
+@pytest.mark.parametrize("rows,batches", [(7, [5, 16]), (33, [6, 17]), (1000, [5, 6, 10, 11, 16, 21, 32, 37]),
+                                          (170001, [9])])
+def test_head_many_tokens_equal_single_tokens(gpu, rows, batches):
+    """Five to sixteen tokens share one pass over the codes (one, two or three
+    tables of columns; 16 tokens a launch, the rest as before): the logits of
+    each token alone, bit for bit, on rows below a tile, past a pair, and past
+    the five tiles that each wave holds at once."""
+    rng = syn.rng_for(1, 6000 + rows)
+    dh = hip.upload_head(gpu, syn.head_chunk(rng, rows, 2048, 0))
+    x = gpu.to_device(syn.rms_normalized(syn.hidden_states(rng, max(batches), 2048)))
+    want = torch.empty((max(batches), rows), dtype=torch.float32, device="cuda")
+    for t in range(max(batches)):
+        hip.head_matmul(gpu, dh, x[t], 1, want[t])
+    for batch in batches:
+        got = torch.full((batch, rows), float("nan"), dtype=torch.float32, device="cuda")
+        hip.head_matmul(gpu, dh, x, batch, got)
+        assert torch.equal(got.view(torch.int32), want[:batch].view(torch.int32)), batch
+
+
 def test_head_argmax_near_ties(gpu, oracle):
     """Rows built to tie or nearly tie with the maximum: the certified
     arg-max must still return the CPU path's first maximum."""

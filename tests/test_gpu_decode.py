@@ -150,6 +150,27 @@ def test_sample_rows_match_oracle(gpu, oracle, temperature, top_p):
     assert got.tolist() == want
 
 
+@pytest.mark.parametrize("temperature,top_p", [(1.0, 0.95), (2.0, 0.999), (1.0, 1.0), (0.5, 0.3)])
+def test_sample_rows_wide_kept_sets(gpu, oracle, temperature, top_p):
+    """Rows whose kept set holds thousands of tokens, so that its end and the
+    draw's token are found by mass: a normal tail under a few likely tokens,
+    normal and nearly flat rows, one with a long run of ties (left to the
+    windows), and draws at both ends."""
+    rng = np.random.default_rng(int(temperature * 100 + top_p * 1000))
+    count = 100003
+    logits = rng.normal(0, 2, (8, count)).astype(np.float32)
+    logits[0:2, rng.integers(0, count, 16)] += 12.0
+    logits[2] = rng.normal(0, 0.05, count)
+    logits[3] = rng.uniform(-1, 1, count)
+    logits[4, 1000:30000] = 0.25
+    logits[5] = rng.normal(0, 8, count)
+    words = rng.integers(0, 2**63, 8, dtype=np.uint64) * 2
+    words[0], words[6], words[7] = 2**64 - 1, 0, 2**64 - 1
+    got = sample_device(gpu, logits, temperature, top_p, words)
+    want = [po.sample_token(oracle, logits[r], temperature, top_p, int(words[r])) for r in range(8)]
+    assert got.tolist() == want
+
+
 def test_sample_rows_small_vocabularies_and_edges(gpu, oracle):
     rng = np.random.default_rng(77)
     for count in (1, 2, 63, 4096, 4097, 12289):

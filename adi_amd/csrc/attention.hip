@@ -60,16 +60,36 @@ struct FullRows {
     float *values[kRowGroup];
 };
 
-// Splits of the history of a row at `tokens` entries: one per 32 entries, at
-// most `cap`. Each row's split count follows from its own position alone, so
-// its result does not depend on the launch's grid (any grid with at least
-// this many splits gives the same bits) or on the other rows.
-__host__ __device__ __forceinline__ uint32_t row_splits(uint32_t tokens, uint32_t cap) {
-    const uint32_t s = (tokens + 31u) / 32u;
-    return s < 1u ? 1u : (s > cap ? cap : s);
+// The parts of a row's history in a decode step over sequences: a part is a
+// block's four waves taking tiles of kTile entries in turn. A row's parts
+// follow from its own position and the step's cap alone, so its result does not
+// depend on the launch's grid (any grid with at least this many parts gives the
+// same bits) or on the other rows. A short history takes one tile a wave, the
+// shortest chain; past kShortHistory entries two tiles a wave, which halves the
+// parts to write and merge (one row at 600 entries: 17.6 us with one tile, 19.9
+// with two; at 4096 28.0 and 24.7; 16 rows at up to 4096 69 and 62).
+constexpr uint32_t kTile = 16;
+constexpr uint32_t kShortHistory = 1024;
+constexpr uint32_t kRowPartials = 1024, kLeastPartials = 64;  // parts of all rows
+__host__ __device__ __forceinline__ uint32_t history_parts(uint32_t tokens) {
+    const uint32_t entries = tokens <= kShortHistory ? 4u * kTile : 8u * kTile;
+    return (tokens + entries - 1u) / entries;
+}
+struct RowParts {
+    uint32_t splits, chunk;  // live parts, entries a part (a multiple of kTile)
+};
+__host__ __device__ __forceinline__ RowParts row_parts(uint32_t tokens, uint32_t cap) {
+    const uint32_t most = history_parts(tokens);
+    const uint32_t splits = most > cap ? cap : most;
+    const uint32_t chunk = ((tokens + splits - 1u) / splits + kTile - 1u) / kTile * kTile;
+    return {(tokens + chunk - 1u) / chunk, chunk};
+}
+// The most parts of a history of 1 .. last entries.
+inline uint32_t most_parts(uint32_t last, uint32_t cap) {
+    return std::min(cap, std::max(history_parts(last), history_parts(std::min(last, kShortHistory))));
 }
 
-// Blocks of the flash-decoding partial kernels (block b runs on XCD b % 8).
+// Blocks of k_attention_partial (block b runs on XCD b % 8).
 // Under kPairSplits splits block b is query head b % 16 of split b / 16: all
 // splits of a head on one XCD, whose L2 then still holds them for the
 // combine. From kPairSplits splits the history is long and the eight query
@@ -232,17 +252,12 @@ __global__ __launch_bounds__(kHeadSize) void k_norm_rope_rows(float *query_gate,
 // accumulator, maximum and denominator to the token's partial rows
 // (maximum -inf and denominator 0 when the split lies past the token).
 // With COHERENT the partial row is written through to memory (a later block
-// of the same launch reads it). The query head is at `query` (global or LDS);
-// entry `fresh` (when below `tokens`) is taken from fresh_key / fresh_value
-// (LDS) instead of the cache.
+// of the same launch reads it). The query head is at `query` (global or LDS).
 template <bool COHERENT = false>
 __device__ __forceinline__ void attention_partial_span(const float *query, const float *keys,
                                                        const float *values, uint32_t tokens,
                                                        uint32_t chunk, float *partial, uint32_t h,
-                                                       uint32_t split, uint32_t splits,
-                                                       uint32_t fresh = 0xFFFFFFFFu,
-                                                       const float *fresh_key = nullptr,
-                                                       const float *fresh_value = nullptr) {
+                                                       uint32_t split, uint32_t splits) {
 #pragma clang fp contract(off)
     __shared__ __align__(16) float wave_acc[4][kHeadSize];
     __shared__ float wave_max[4], wave_den[4];
@@ -259,9 +274,8 @@ __device__ __forceinline__ void attention_partial_span(const float *query, const
     // its dot products reduced together, then the online updates in order
     constexpr uint32_t kBatch = 8;
     for (uint32_t t0 = begin + wave; t0 < end; t0 += 4u * kBatch) {
-        // every entry from the cache, with no branch around a load (so the
-        // batch's loads are counted and waited for once); the fresh entry's
-        // cache slot is read too and then replaced by its LDS copy
+        // no branch around a load, so that the batch's loads are counted and
+        // waited for once
         float4 k[kBatch], v[kBatch];
 #pragma unroll
         for (uint32_t j = 0; j < kBatch; ++j) {
@@ -269,14 +283,6 @@ __device__ __forceinline__ void attention_partial_span(const float *query, const
             const size_t at = (static_cast<size_t>(t) * kKvHeads + kv) * kHeadSize;
             k[j] = reinterpret_cast<const float4 *>(keys + at)[lane];
             v[j] = reinterpret_cast<const float4 *>(values + at)[lane];
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < kBatch; ++j) {
-            const uint32_t t = t0 + 4u * j < end ? t0 + 4u * j : t0;
-            if (t == fresh) {  // wave-uniform
-                k[j] = reinterpret_cast<const float4 *>(fresh_key)[lane];
-                v[j] = reinterpret_cast<const float4 *>(fresh_value)[lane];
-            }
         }
         float dot[kBatch];
 #pragma unroll
@@ -342,29 +348,234 @@ __global__ __launch_bounds__(256) void k_attention_partial(const float *query_ga
                            pb.split, splits);
 }
 
-// Row r of a decode step over sequences sees its own cache's entries
-// 0 .. positions[r], split evenly over row_splits(positions[r] + 1, cap)
-// splits; the grid's further splits lie past the row's tokens and come out
-// empty (skipped by the combine).
-__global__ __launch_bounds__(256) void k_attention_partial_rows(const float *query_gate,
-                                                                FullRows rows,
-                                                                const uint32_t *positions,
-                                                                uint32_t cap, uint32_t grid_splits,
-                                                                float *partial) {
-    const PartialBlock pb = partial_block(blockIdx.x, grid_splits);
-    if (!pb.live) {
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr uint32_t kHeadsPerKv = kQueryHeads / kKvHeads;  // 8
+constexpr uint32_t kQueryPad = kHeadSize + 16;  // LDS rows whose 16-byte pieces fall on different banks
+constexpr uint32_t kMergePad = kHeadSize + 4;
+
+struct RowsLds {
+    __align__(16) float query[kHeadsPerKv][kQueryPad];
+    __align__(16) float acc[4][kHeadsPerKv][kMergePad];
+    float maximum[4][kHeadsPerKv], denominator[4][kHeadsPerKv];
+    uint32_t odd;
+};
+
+// Entries [split * chunk, ...) below `tokens` of KV head `kv` for its eight
+// query heads (lds.query) by a block of four waves, wave w taking every fourth
+// tile of kTile entries, and the split's part of each head to partial (written
+// through to memory with COHERENT: a later block of the same launch reads it).
+//
+// A tile is two chains of v_mfma_f32_16x16x4_f32 in which a lane's registers
+// are loaded as the matrix core reads them, straight from the cache: the
+// scores are keys (16 entries a column of A, dimensions 16 j + 4 g + i at step
+// (j, i) of lane group g) times queries (B, the eight heads twice), and their
+// result, entry 4 g + r of head l % 16 in register r, is B of the second
+// chain's step r as it stands; its A is the values transposed (dimension
+// 64 m + 4 (l % 16) + i of entry 4 g + r). So a head's maximum, factors and
+// weights live in the lanes of its column, one exponential serves one score,
+// and an entry is read once for the eight heads.
+//
+// Bound by the entries' bytes where rows and histories are many, by a part's
+// chain of norm, tile and merge where they are few. One head's wave at a time
+// over float registers (a wave sum and an exponential a head and entry, each
+// entry read eight times) took 201 us for 32 rows at up to 2,000 entries, this
+// 62 (131 MB: 2.1 TB/s), and one row at 2,000 27.1 and 21.3.
+template <bool COHERENT>
+__device__ __forceinline__ void attention_rows_span(RowsLds &lds, const float *keys, const float *values,
+                                                    uint32_t tokens, uint32_t chunk, float *partial, uint32_t kv,
+                                                    uint32_t split, uint32_t splits) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t c = lane & 15u, g = lane >> 4;
+    const uint32_t begin = split * chunk;
+    const uint32_t end = begin + chunk < tokens ? begin + chunk : tokens;
+    const float *key_head = keys + static_cast<size_t>(kv) * kHeadSize;
+    const float *value_head = values + static_cast<size_t>(kv) * kHeadSize;
+    constexpr size_t kEntry = kKvHeads * kHeadSize;
+    const float *query = lds.query[c & 7u] + 4u * g;
+    f32x4 k[16], v[16], o[16];
+    // entries past the part read its last one; their scores are masked
+    const auto load_keys = [&](uint32_t t0) {
+        const uint32_t t = t0 + c < end ? t0 + c : end - 1u;
+        const float *at = key_head + t * kEntry + 4u * g;
+#pragma unroll
+        for (uint32_t j = 0; j < 16; ++j) {
+            k[j] = *reinterpret_cast<const f32x4 *>(at + 16u * j);
+        }
+    };
+    const auto load_values = [&](uint32_t t0) {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            const uint32_t e = t0 + 4u * g + r;
+            const float *at = value_head + (e < end ? e : end - 1u) * kEntry + 4u * c;
+#pragma unroll
+            for (uint32_t m = 0; m < 4; ++m) {
+                v[4u * r + m] = *reinterpret_cast<const f32x4 *>(at + 64u * m);
+            }
+        }
+    };
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) {
+        o[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    float maximum = -__builtin_huge_valf(), denominator = 0.0f;
+    bool odd = false;
+    uint32_t t0 = begin + wave * kTile;
+    if (t0 < end) {
+        load_keys(t0);
+        load_values(t0);
+    }
+    for (; t0 < end; t0 += 4u * kTile) {
+        const bool ragged = t0 + kTile >= tokens;  // the row's last tile
+        f32x4 s[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            s[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 16; ++j) {
+            const f32x4 q = *reinterpret_cast<const f32x4 *>(query + 16u * j);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j][i], q[i], s[i], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (t0 + 4u * kTile < end) {
+            load_keys(t0 + 4u * kTile);
+        }
+        f32x4 p = ((s[0] + s[1]) + (s[2] + s[3])) * (1.0f / 16.0f);  // 1 / sqrt(256)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            odd |= !(fabsf(p[r]) < __builtin_huge_valf());
+        }
+        if (ragged) {
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) {
+                const uint32_t e = t0 + 4u * g + r;
+                p[r] = e < tokens ? p[r] : -__builtin_huge_valf();
+#pragma unroll
+                for (uint32_t m = 0; m < 4; ++m) {
+                    v[4u * r + m] = e < tokens ? v[4u * r + m] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+            }
+        }
+        float top = fmaxf(fmaxf(p[0], p[1]), fmaxf(p[2], p[3]));
+        top = fmaxf(top, lane_xor<16>(top));
+        top = fmaxf(top, lane_xor<32>(top));
+        if (__any(top > maximum)) {
+            const float next = fmaxf(top, maximum);
+            const float factor = expf(maximum - next);
+            maximum = next;
+            denominator *= factor;
+#pragma unroll
+            for (uint32_t i = 0; i < 16; ++i) {
+                o[i] *= factor;
+            }
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            p[r] = expf(p[r] - maximum);
+        }
+        denominator += (p[0] + p[1]) + (p[2] + p[3]);
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+#pragma unroll
+            for (uint32_t m = 0; m < 4; ++m) {
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    o[4u * m + i] =
+                        __builtin_amdgcn_mfma_f32_16x16x4f32(v[4u * r + m][i], p[r], o[4u * m + i], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (t0 + 4u * kTile < end) {
+            load_values(t0 + 4u * kTile);
+        }
+    }
+    denominator += lane_xor<16>(denominator);
+    denominator += lane_xor<32>(denominator);
+    if (threadIdx.x == 0) {
+        lds.odd = 0u;
+    }
+    __syncthreads();
+    if (__any(odd) && lane == 0) {
+        lds.odd = 1u;
+    }
+    if (c < kHeadsPerKv) {
+#pragma unroll
+        for (uint32_t m = 0; m < 4; ++m) {
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) {
+                *reinterpret_cast<f32x4 *>(&lds.acc[wave][c][64u * m + 16u * g + 4u * r]) =
+                    f32x4{o[4u * m][r], o[4u * m + 1u][r], o[4u * m + 2u][r], o[4u * m + 3u][r]};
+            }
+        }
+        if (g == 0u) {
+            lds.maximum[wave][c] = maximum;
+            lds.denominator[wave][c] = denominator;
+        }
+    }
+    __syncthreads();
+    if (lds.odd != 0u) {  // uniform: a score that is not a number, head by head
+        for (uint32_t h = 0; h < kHeadsPerKv; ++h) {
+            attention_partial_span<COHERENT>(lds.query[h], keys, values, tokens, chunk, partial,
+                                             kv * kHeadsPerKv + h, split, splits);
+            __syncthreads();
+        }
         return;
     }
-    const uint32_t r = blockIdx.z;
-    const uint32_t tokens = positions[r] + 1;
-    const uint32_t splits = row_splits(tokens, cap);
-    attention_partial_span(query_gate + static_cast<size_t>(r) * kQueryHeads * kQueryStride +
-                               static_cast<size_t>(pb.head) * kQueryStride,
-                           rows.keys[r], rows.values[r], tokens, (tokens + splits - 1u) / splits,
-                           partial + static_cast<size_t>(r) * kQueryHeads * grid_splits * kPartialStride,
-                           pb.head, pb.split, grid_splits);
+#pragma unroll
+    for (uint32_t h = 0; h < kHeadsPerKv; ++h) {
+        float m = lds.maximum[0][h];
+        for (uint32_t w = 1; w < 4; ++w) {
+            m = fmaxf(m, lds.maximum[w][h]);
+        }
+        float a = 0.0f, d = 0.0f;
+        if (m != -__builtin_huge_valf()) {  // else no token in this split
+            for (uint32_t w = 0; w < 4; ++w) {
+                const float f = expf(lds.maximum[w][h] - m);  // 0 for a wave without tokens
+                a += lds.acc[w][h][threadIdx.x] * f;
+                d += lds.denominator[w][h] * f;
+            }
+        }
+        float *out = partial + (static_cast<size_t>(kv * kHeadsPerKv + h) * splits + split) * kPartialStride;
+        if constexpr (COHERENT) {
+            coherent_store(out + threadIdx.x, a);
+            if (threadIdx.x == 0) {
+                coherent_store(out + kHeadSize, m);
+                coherent_store(out + kHeadSize + 1, d);
+            }
+        } else {
+            out[threadIdx.x] = a;
+            if (threadIdx.x == 0) {
+                out[kHeadSize] = m;
+                out[kHeadSize + 1] = d;
+            }
+        }
+    }
 }
 
+// Row r of a decode step over sequences sees its own cache's entries
+// 0 .. positions[r] in row_parts' parts: block (KV head, split, r). The grid's
+// further splits lie past the row's tokens and come out empty (skipped by the
+// combine).
+__global__ __launch_bounds__(256, 2) void k_attention_partial_rows(const float *query_gate, FullRows rows,
+                                                                   const uint32_t *positions, uint32_t cap,
+                                                                   uint32_t grid_splits, float *partial) {
+    __shared__ RowsLds lds;
+    const uint32_t kv = blockIdx.x % kKvHeads, split = blockIdx.x / kKvHeads, r = blockIdx.z;
+    const uint32_t tokens = positions[r] + 1;
+    const RowParts parts = row_parts(tokens, cap);
+    for (uint32_t h = 0; h < kHeadsPerKv; ++h) {
+        lds.query[h][threadIdx.x] =
+            query_gate[(static_cast<size_t>(r) * kQueryHeads + kv * kHeadsPerKv + h) * kQueryStride + threadIdx.x];
+    }
+    __syncthreads();
+    attention_rows_span<false>(lds, rows.keys[r], rows.values[r], tokens, parts.chunk,
+                               partial + static_cast<size_t>(r) * kQueryHeads * grid_splits * kPartialStride, kv,
+                               split, grid_splits);
+}
 // The splits of one query head merged (splits <= N): every split's
 // accumulator, then the splits' maxima and denominators (through LDS),
 // loaded in one round, then the accumulators added in split order.
@@ -433,88 +644,150 @@ __global__ __launch_bounds__(kHeadSize) void k_attention_combine(const float *pa
     attended[static_cast<size_t>(h) * kHeadSize + t] = a * (1.0f / d) * sigmoid_of(gate);
 }
 
+// norm_rope_head by one wave, the same sums: lane l holds dimensions l, l + 64,
+// l + 128, l + 192; row holds the position's 32 cosines and 32 sines.
+__device__ __forceinline__ void norm_rope_wave(const float *src, float *dst, const uint16_t *w, const float *row) {
+#pragma clang fp contract(off)
+    const uint32_t lane = threadIdx.x & 63u;
+    float x[4], weight[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        x[i] = src[64u * i + lane];
+        weight[i] = bf16_bits_to_float(w[64u * i + lane]);
+    }
+    const float cosine = row[lane & 31u], sine = row[kRopeHalf + (lane & 31u)];
+    float squares = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        squares += wave_sum(x[i] * x[i]);
+    }
+    const float scale = 1.0f / sqrtf(squares / static_cast<float>(kHeadSize) + kEpsilon);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        x[i] *= scale * (1.0f + weight[i]);
+    }
+    const float other = lane_xor<32>(x[0]);
+    x[0] = lane < kRopeHalf ? x[0] * cosine - other * sine : x[0] * cosine + other * sine;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        dst[64u * i + lane] = x[i];
+    }
+}
+
 // One decode token of each of up to kRowGroup sequences through full
 // attention's core in one launch, with the arithmetic of k_norm_rope_rows,
-// k_attention_partial_rows and k_attention_combine. Block (query head h,
-// split, sequence r), dealt as partial_block deals them:
-// - normalizes and rotates its query head into LDS itself (every split of a
-//   head does);
-// - the splits holding the row's new entry (position) normalize and rotate
-//   its key and take its value themselves, and one of them per KV head (the
-//   first query head of the KV head) writes both into the cache: no block
-//   reads that entry from the cache;
-// - writes its split's partial row through to memory; the last block of the
-//   head's grid_splits through the head's ticket merges them and applies the
-//   sigmoid gate.
-// `tickets` holds kQueryHeads words a sequence, zero between calls.
-__global__ __launch_bounds__(256) void k_attention_rows_one(const float *query_gate, const float *key,
-                                                            const float *value, const uint16_t *query_norm,
-                                                            const uint16_t *key_norm, const float *rope_rows,
-                                                            FullRows rows, const uint32_t *positions,
-                                                            uint32_t cap, uint32_t grid_splits, float *partial,
-                                                            float *attended, uint32_t *tickets) {
-    __shared__ float sums[16];
-    __shared__ float head[kHeadSize];
-    __shared__ __align__(16) float q_lds[kHeadSize];
-    __shared__ __align__(16) float key_lds[kHeadSize];
-    __shared__ __align__(16) float value_lds[kHeadSize];
-    __shared__ float split_max[kMaxSplits], split_den[kMaxSplits], split_factor[kMaxSplits];
+// k_attention_partial_rows and k_attention_combine. Block (KV head, split,
+// sequence r):
+// - normalizes and rotates its eight query heads into LDS itself (every split
+//   does);
+// - the split holding the row's new entry (position) normalizes and rotates its
+//   key and writes it and the value into the cache: no other block reads that
+//   entry;
+// - writes its split's partial rows through to memory; the last block of the
+//   row's live splits through the KV head's ticket merges the eight heads and
+//   applies the sigmoid gates.
+// Blocks of splits past the row's history leave at once. `tickets` holds
+// kQueryHeads words a sequence (one a KV head used), zero between calls.
+__global__ __launch_bounds__(256, 2) void k_attention_rows_one(const float *query_gate, const float *key,
+                                                               const float *value, const uint16_t *query_norm,
+                                                               const uint16_t *key_norm, const float *rope_rows,
+                                                               FullRows rows, const uint32_t *positions, uint32_t cap,
+                                                               uint32_t grid_splits, float *partial, float *attended, uint32_t *tickets) {
+#pragma clang fp contract(off)
+    __shared__ RowsLds lds;
     __shared__ uint32_t last;
-    const PartialBlock pb = partial_block(blockIdx.x, grid_splits);
-    if (!pb.live) {
-        return;
-    }
-    const uint32_t r = blockIdx.z, t = threadIdx.x;
-    const uint32_t h = pb.head, split = pb.split, kv = h / (kQueryHeads / kKvHeads);
+    const uint32_t kv = blockIdx.x % kKvHeads, split = blockIdx.x / kKvHeads, r = blockIdx.z;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     const uint32_t position = positions[r];
     const uint32_t tokens = position + 1u;
-    const uint32_t splits = row_splits(tokens, cap);
-    const uint32_t chunk = (tokens + splits - 1u) / splits;
-    const uint32_t begin = split * chunk;
-    const bool fresh = begin <= position && position < begin + chunk;  // uniform over the block
-    const float *qg = query_gate + (static_cast<size_t>(r) * kQueryHeads + h) * kQueryStride;
-    float cosine = 0.0f, sine = 0.0f;
-    if (t < kRopeHalf) {
-        const float *row = rope_rows + static_cast<size_t>(position) * (2 * kRopeHalf);
-        cosine = row[t];
-        sine = row[kRopeHalf + t];
+    const RowParts parts = row_parts(tokens, cap);
+    if (split >= parts.splits) {  // uniform over the block
+        return;
     }
-    norm_rope_head(qg, q_lds, query_norm, cosine, sine, sums, head);
-    if (fresh) {
-        __syncthreads();  // head[] is free again
+    const float *rope = rope_rows + static_cast<size_t>(position) * (2 * kRopeHalf);
+    const size_t head = static_cast<size_t>(r) * kQueryHeads + kv * kHeadsPerKv;
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+        const uint32_t h = 2u * wave + i;
+        norm_rope_wave(query_gate + (head + h) * kQueryStride, lds.query[h], query_norm, rope);
+    }
+    if (split == parts.splits - 1u) {  // uniform over the block
         const size_t src = (static_cast<size_t>(r) * kKvHeads + kv) * kHeadSize;
-        norm_rope_head(key + src, key_lds, key_norm, cosine, sine, sums, head);
-        value_lds[t] = value[src + t];
-        __syncthreads();
-        if (h % (kQueryHeads / kKvHeads) == 0u) {
-            const size_t entry = (static_cast<size_t>(position) * kKvHeads + kv) * kHeadSize;
-            rows.keys[r][entry + t] = key_lds[t];
-            rows.values[r][entry + t] = value_lds[t];
+        const size_t entry = (static_cast<size_t>(position) * kKvHeads + kv) * kHeadSize;
+        if (wave == 0u) {
+            norm_rope_wave(key + src, rows.keys[r] + entry, key_norm, rope);
         }
+        rows.values[r][entry + t] = value[src + t];
     }
-    __syncthreads();
+    __syncthreads();  // the block reads back its own entry
     float *p = partial + static_cast<size_t>(r) * kQueryHeads * grid_splits * kPartialStride;
-    attention_partial_span<true>(q_lds, rows.keys[r], rows.values[r], tokens, chunk, p, h, split, grid_splits,
-                                 position, key_lds, value_lds);
+    attention_rows_span<true>(lds, rows.keys[r], rows.values[r], tokens, parts.chunk, p, kv, split, grid_splits);
     wait_stores();
     __syncthreads();
-    uint32_t *ticket = tickets + static_cast<size_t>(r) * kQueryHeads + h;
+    uint32_t *ticket = tickets + static_cast<size_t>(r) * kQueryHeads + kv;
     if (t == 0) {
-        last = coherent_add(ticket, 1u) + 1u == grid_splits ? 1u : 0u;
+        last = coherent_add(ticket, 1u) + 1u == parts.splits ? 1u : 0u;
     }
     __syncthreads();
     if (last == 0u) {
         return;
     }
-    const float gate = qg[kHeadSize + t];
-    const float *ph = p + static_cast<size_t>(h) * grid_splits * kPartialStride;
-    float a, d;
-    if (grid_splits <= 16u) {
-        combine_splits<16, true>(ph, grid_splits, t, split_max, split_den, split_factor, a, d);
-    } else {
-        combine_splits<kMaxSplits, true>(ph, grid_splits, t, split_max, split_den, split_factor, a, d);
+    // k_attention_combine's sums, two heads a wave: lane s holds split s's
+    // maximum and denominator, lane l dimensions l + 64 i
+    static_assert(kMaxSplits <= 64, "a lane a split");
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+        const uint32_t h = 2u * wave + i;
+        const float *ph = p + static_cast<size_t>(kv * kHeadsPerKv + h) * grid_splits * kPartialStride;
+        float mx = -__builtin_huge_valf(), den = 0.0f;
+        if (lane < parts.splits) {
+            mx = coherent_load(ph + lane * kPartialStride + kHeadSize);
+            den = coherent_load(ph + lane * kPartialStride + kHeadSize + 1);
+        }
+        float gate[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            gate[j] = query_gate[(head + h) * kQueryStride + kHeadSize + 64u * j + lane];
+        }
+        float m = mx;
+        m = fmaxf(m, lane_xor<1>(m));
+        m = fmaxf(m, lane_xor<2>(m));
+        m = fmaxf(m, lane_xor<4>(m));
+        m = fmaxf(m, lane_xor<8>(m));
+        m = fmaxf(m, lane_xor<16>(m));
+        m = fmaxf(m, lane_xor<32>(m));
+        const float factor = expf(mx - m);
+        float a[4] = {0.0f, 0.0f, 0.0f, 0.0f}, d = 0.0f;
+        constexpr uint32_t kBatch = 8;
+        for (uint32_t s0 = 0; s0 < parts.splits; s0 += kBatch) {
+            float acc[kBatch][4];
+#pragma unroll
+            for (uint32_t s = 0; s < kBatch; ++s) {
+                const uint32_t at = s0 + s < parts.splits ? s0 + s : parts.splits - 1u;
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    acc[s][j] = coherent_load(ph + at * kPartialStride + 64u * j + lane);
+                }
+            }
+#pragma unroll
+            for (uint32_t s = 0; s < kBatch; ++s) {
+                const int at = static_cast<int>(s0 + s);
+                const float ds = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(den), at & 63));
+                const float fs = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(factor), at & 63));
+                if (s0 + s < parts.splits && ds != 0.0f) {  // uniform
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        a[j] += acc[s][j] * fs;
+                    }
+                    d += ds * fs;
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            attended[(head + h) * kHeadSize + 64u * j + lane] = a[j] * (1.0f / d) * sigmoid_of(gate[j]);
+        }
     }
-    attended[(static_cast<size_t>(r) * kQueryHeads + h) * kHeadSize + t] = a * (1.0f / d) * sigmoid_of(gate);
     if (t == 0) {
         coherent_store(ticket, 0u);
     }
@@ -1424,13 +1697,18 @@ void full_attention_rows(adi_hip_context *ctx, const adi_hip_full_attention *L, 
     last = span > last ? span : last;
     auto &ws = ctx->layer_workspace;
     ws.used = 0;
-    const uint32_t cap = kMaxSplits / rows > 0 ? kMaxSplits / rows : 1u;
-    const uint32_t splits = row_splits(last, cap);
     const size_t n = rows;
-    ws.ensure(Workspace::round(n * kQueryHeads * kQueryStride * 4) +
-              Workspace::round(n * kKvHeads * kHeadSize * 4) * 2 +
-              Workspace::round(n * kQueryHeads * kHeadSize * 4) +
-              Workspace::round(n * kQueryHeads * splits * kPartialStride * 4));
+    const size_t fixed = Workspace::round(n * kQueryHeads * kQueryStride * 4) +
+                         Workspace::round(n * kKvHeads * kHeadSize * 4) * 2 +
+                         Workspace::round(n * kQueryHeads * kHeadSize * 4);
+    // partial rows of at most kRowPartials parts, and within a workspace limit
+    // (kLeastPartials parts are asked for in any case)
+    const size_t part = n * kQueryHeads * kPartialStride * 4;
+    const size_t fit = ws.limit > fixed + 256 ? (ws.limit - fixed - 256) / part : 0;
+    uint32_t cap = std::min<uint32_t>(kMaxSplits, kRowPartials / rows);
+    cap = std::max<uint32_t>(std::min<size_t>(cap, fit), std::max<uint32_t>(kLeastPartials / rows, 1u));
+    const uint32_t splits = most_parts(last, cap);
+    ws.ensure(fixed + Workspace::round(part * splits));
     float *query_gate = ws.take<float>(n * kQueryHeads * kQueryStride);
     float *key = ws.take<float>(n * kKvHeads * kHeadSize);
     float *value = ws.take<float>(n * kKvHeads * kHeadSize);
@@ -1450,7 +1728,7 @@ void full_attention_rows(adi_hip_context *ctx, const adi_hip_full_attention *L, 
         if (ctx->fused_moe) {
             static_assert(kRowGroup * kQueryHeads <= kMoeSyncWords - kMoeSyncAttention,
                           "the attention tickets fit their sync line");
-            launch(ctx, "attention_rows_one", k_attention_rows_one, dim3(partial_blocks(splits), 1, count),
+            launch(ctx, "attention_rows_one", k_attention_rows_one, dim3(kKvHeads * splits, 1, count),
                    dim3(256), 0, static_cast<const float *>(qg),
                    static_cast<const float *>(key + static_cast<size_t>(first) * kKvHeads * kHeadSize),
                    static_cast<const float *>(value + static_cast<size_t>(first) * kKvHeads * kHeadSize),
@@ -1466,7 +1744,7 @@ void full_attention_rows(adi_hip_context *ctx, const adi_hip_full_attention *L, 
                static_cast<const float *>(value + static_cast<size_t>(first) * kKvHeads * kHeadSize),
                L->query_norm, L->key_norm, rope, table, row_positions);
         launch(ctx, "attention_partial_rows", k_attention_partial_rows,
-               dim3(partial_blocks(splits), 1, count), dim3(256), 0, static_cast<const float *>(qg), table,
+               dim3(kKvHeads * splits, 1, count), dim3(256), 0, static_cast<const float *>(qg), table,
                row_positions, cap, splits,
                partial + static_cast<size_t>(first) * kQueryHeads * splits * kPartialStride);
         launch(ctx, "attention_combine", k_attention_combine, dim3(kQueryHeads, count), dim3(kHeadSize), 0,

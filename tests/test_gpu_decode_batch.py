@@ -189,6 +189,62 @@ def test_decode_batch_long_histories(gpu, parts):
         assert max_rel_error(one[b], logits.cpu().numpy()) <= 1e-3, b
 
 
+@pytest.mark.parametrize("limit", [None, 4096])
+def test_decode_batch_history_edges(gpu, parts, limit):
+    """Rows whose histories end at the edges of the attention's tiles of 16
+    entries and parts of 64 and 128, one with a key whose scores overflow (a
+    single dimension: infinities of either sign or huge, no NaN), with partial
+    rows for every part and (limit: parts of all rows) at the least workspace.
+    The logits are bit-identical with the one-launch paths off and within 1e-3
+    of the same token through the one-token chunk kernels."""
+    model = parts["one"]
+    positions = [0, 14, 15, 16, 62, 63, 64, 127, 1022, 1023, 1024, 1151, 1152, 1300, 41, 40]
+    n = len(positions)
+    tokens = [(7 * i + 3) % VOCAB for i in range(n)]
+
+    def sequences():
+        g = torch.Generator(device="cuda").manual_seed(5)
+        seqs = [hip.Sequence(model, p + 1) for p in positions]
+        for s, p in zip(seqs, positions):
+            for t in s.tensors[3]:
+                t[:p] = torch.randn(t[:p].shape, generator=g, device="cuda")
+            s.struct.position = p
+        for i, huge in ((-2, 1e37), (-1, 3e38)):
+            seqs[i].tensors[3][0][5] = 0.0
+            seqs[i].tensors[3][0][5, :, 200] = huge
+        torch.cuda.synchronize()
+        return seqs
+
+    def run(ctx, fused):
+        ctx.set_fused_decode(fused)
+        try:
+            seqs = sequences()
+            print("decode_batch edges", limit, fused, flush=True)
+            out = torch.empty((n, VOCAB), dtype=torch.float32, device="cuda")
+            hip.decode_batch(ctx, model, tokens, seqs, out)
+            ctx.synchronize()
+            return out.cpu().numpy()
+        finally:
+            ctx.set_fused_decode(True)
+
+    run(gpu, True)  # the arenas hold the full number of parts
+    if limit:
+        gpu.set_workspace_limit(limit)
+    try:
+        one, separate = run(gpu, True), run(gpu, False)
+    finally:
+        gpu.set_workspace_limit(None)
+    assert np.array_equal(one.view(np.uint32), separate.view(np.uint32))
+    for b, (s, token) in enumerate(zip(sequences(), tokens)):
+        logits = torch.empty(VOCAB, dtype=torch.float32, device="cuda")
+        hip.prefill(gpu, model, [token], s, logits)
+        want = logits.cpu().numpy()
+        if b == n - 1:
+            assert np.array_equal(np.isfinite(one[b]), np.isfinite(want))
+        else:
+            assert np.isfinite(want).all() and max_rel_error(one[b], want) <= 1e-3, (b, positions[b])
+
+
 def test_fresh_sequences_batched_equal_decoded_alone(gpu, parts):
     """tests/model_batch_test.cpp:24-51: two new sequences decoded as one
     batch give the logits of each decoded alone, and both reach position 1.

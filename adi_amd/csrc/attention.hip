@@ -1102,14 +1102,14 @@ __device__ __forceinline__ ConvChannel conv_channel(const float *qkv_row, const 
 // norms, the delta rule and the gated RMS norm (src/executor.cpp:480-550),
 // with the arithmetic of k_linear_conv_rows, k_gated_delta_rows and
 // k_linear_norm_gate. Block (value head h, row block y, sequence r):
-// - convolves the 128 query and 128 key channels of h's key head itself (the
-//   16 blocks of a key head each do, each sum in the 128-thread block's
-//   order) and its own 16 value channels, whose state only it shifts;
-// - updates its 16 state rows and writes their outputs through to memory;
-// - the last of the head's 8 blocks through the head's ticket reads the 128
-//   outputs back and writes the head's gated norm; the last of the key
-//   head's 16 blocks through its ticket shifts the query and key channels'
-//   state (every one of them has read it by then).
+// - convolves the 128 query and 128 key channels of h's key head itself (every
+//   block of a key head does, each sum in the 128-thread block's order) and its
+//   own ROWS value channels, whose state only it shifts;
+// - updates its ROWS state rows and writes their outputs through to memory;
+// - the last of the head's blocks through the head's ticket reads the 128
+//   outputs back and writes the head's gated norm; the last of the key head's
+//   blocks through its ticket shifts the query and key channels' state (every
+//   one of them has read it by then).
 // `tickets` holds 48 words a sequence (32 value heads, 16 key heads), zero
 // between calls: the last block through each ticket clears it.
 // With LANES 8 or 16 the block also computes its head's alpha and beta
@@ -1117,8 +1117,17 @@ __device__ __forceinline__ ConvChannel conv_channel(const float *qkv_row, const 
 // as k_bf16_lds does): the row and the two weight rows staged in LDS, one
 // wave's lanes 0 .. 2 LANES - 1 running the chains. With LANES 0 they come
 // precomputed in alpha and beta.
+//
+// ROWS state rows a block: every block of a head repeats the head's
+// convolution, decay chains and their loads, so more rows a block cost less in
+// all, and fewer blocks leave the chip idle for few sequences. us a launch with
+// 16, 32, 64, 128 rows: 1 sequence 11.0, 9.9, 11.1, 13.0; 4 15.4, 13.0, 13.0,
+// 14.3; 8 20.4, 17.1, 16.8, 17.3; 16 32.9, 26.7, 23.3, 23.3; 32 (134 MB of
+// states) 54.3, 40.8, 40.3, 42.6.
+constexpr uint32_t kCoreRows = 32;       // below kCoreManyRows sequences, then 64
+constexpr uint32_t kCoreManyRows = 8;
 constexpr uint32_t kDecayColumns = 2048;  // the widest row staged for alpha and beta
-template <int LANES>
+template <int LANES, uint32_t ROWS>
 __global__ __launch_bounds__(256) void k_linear_core_rows(const float *qkv, const uint16_t *weights,
                                                           LinearRows rows, const float *x,
                                                           const uint16_t *alpha_w, const uint16_t *beta_w,
@@ -1128,11 +1137,11 @@ __global__ __launch_bounds__(256) void k_linear_core_rows(const float *qkv, cons
                                                           const float *gate, float *recurrent_output,
                                                           float *normalized, uint32_t *tickets) {
 #pragma clang fp contract(off)
-    constexpr uint32_t kRows = kDeltaRows / 4u;
-    constexpr uint32_t kHeadBlocks = kLinearHead / kDeltaRows;
+    constexpr uint32_t kRows = ROWS / 4u;
+    constexpr uint32_t kHeadBlocks = kLinearHead / ROWS;
     constexpr uint32_t kStaged = LANES > 0 ? kDecayColumns : 4u;
     __shared__ float qk[2][kLinearHead];
-    __shared__ float vv[kDeltaRows];
+    __shared__ float vv[ROWS];
     __shared__ float part[4];
     __shared__ float decay_in[2];
     __shared__ __align__(16) float x_lds[kStaged];
@@ -1143,7 +1152,7 @@ __global__ __launch_bounds__(256) void k_linear_core_rows(const float *qkv, cons
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     const float *row = qkv + static_cast<size_t>(r) * kChannels;
     float *history = rows.convolution[r];
-    const uint32_t row0 = y * kDeltaRows + wave * kRows;
+    const uint32_t row0 = y * ROWS + wave * kRows;
     // the state rows first, so that their loads overlap the convolution
     float2 *state = reinterpret_cast<float2 *>(rows.recurrent[r] +
                                                (static_cast<size_t>(h) * kLinearHead + row0) * kLinearHead);
@@ -1197,8 +1206,8 @@ __global__ __launch_bounds__(256) void k_linear_core_rows(const float *qkv, cons
     if (lane == 0) {
         part[wave] = sq;
     }
-    if (t < kDeltaRows) {
-        const uint32_t cv = 2u * kQkSize + h * kLinearHead + y * kDeltaRows + t;
+    if (t < ROWS) {
+        const uint32_t cv = 2u * kQkSize + h * kLinearHead + y * ROWS + t;
         float *hv = history + static_cast<size_t>(cv) * 3u;
         const ConvChannel v = conv_channel(row, weights, hv, cv);
         vv[t] = v.y;
@@ -1240,7 +1249,7 @@ __global__ __launch_bounds__(256) void k_linear_core_rows(const float *qkv, cons
         const float softplus = biased > 20.0f ? biased : log1pf(expf(biased));
         const float decay = expf(-rate * softplus);
         float *out = recurrent_output + static_cast<size_t>(r) * kValueSize + static_cast<size_t>(h) * kLinearHead;
-        float attended[kRows];  // the rows' chains in one block of code
+        float attended = 0.0f;  // lane j the output of row j
 #pragma unroll
         for (uint32_t j = 0; j < kRows; ++j) {
             s[j].x *= decay;
@@ -1249,13 +1258,11 @@ __global__ __launch_bounds__(256) void k_linear_core_rows(const float *qkv, cons
             const float delta = (vv[wave * kRows + j] - prediction) * beta_value;
             s[j].x += k.x * delta;
             s[j].y += k.y * delta;
-            attended[j] = wave_sum(s[j].x * q.x + s[j].y * q.y) * output_scale;
+            const float output = wave_sum(s[j].x * q.x + s[j].y * q.y) * output_scale;
+            attended = lane == j ? output : attended;
         }
-        if (lane == 0) {
-#pragma unroll
-            for (uint32_t j = 0; j < kRows; ++j) {
-                coherent_store(out + row0 + j, attended[j]);
-            }
+        if (lane < kRows) {
+            coherent_store(out + row0 + lane, attended);
         }
 #pragma unroll
         for (uint32_t j = 0; j < kRows; ++j) {
@@ -1513,11 +1520,17 @@ void launch_linear_core(adi_hip_context *ctx, const adi_hip_linear_attention *L,
     using Kernel = void (*)(const float *, const uint16_t *, LinearRows, const float *, const uint16_t *,
                             const uint16_t *, uint32_t, const float *, const float *, const uint16_t *,
                             const uint16_t *, const uint16_t *, const float *, float *, float *, uint32_t *);
-    Kernel kernel = k_linear_core_rows<0>;
-    if (core_takes_decay(ctx, L, x)) {
-        kernel = ctx->isa_lanes == 16 ? k_linear_core_rows<16> : k_linear_core_rows<8>;
-    }
-    launch(ctx, "linear_core", kernel, dim3(kValueHeads, kLinearHead / kDeltaRows, count), dim3(256), 0, qkv,
+    const uint32_t lanes = core_takes_decay(ctx, L, x) ? ctx->isa_lanes : 0u;
+    const auto pick = [&](auto rows) -> Kernel {
+        constexpr uint32_t kBlockRows = decltype(rows)::value;
+        return lanes == 16u  ? k_linear_core_rows<16, kBlockRows>
+               : lanes == 8u ? k_linear_core_rows<8, kBlockRows>
+                             : k_linear_core_rows<0, kBlockRows>;
+    };
+    const uint32_t block_rows = count < kCoreManyRows ? kCoreRows : 2u * kCoreRows;
+    const Kernel kernel = count < kCoreManyRows ? pick(std::integral_constant<uint32_t, kCoreRows>{})
+                                                : pick(std::integral_constant<uint32_t, 2u * kCoreRows>{});
+    launch(ctx, "linear_core", kernel, dim3(kValueHeads, kLinearHead / block_rows, count), dim3(256), 0, qkv,
            L->convolution, table, x, L->alpha.values, L->beta.values, L->alpha.columns, alpha, beta,
            L->alpha_bias, L->a_log, L->norm, gate, recurrent_output, normalized, ctx->moe_sync + kMoeSyncLinear);
 }

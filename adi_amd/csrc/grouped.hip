@@ -959,6 +959,207 @@ __global__ __launch_bounds__(kNeThreads) void k_ne_mfma(NeMfmaJobs J) {
     }
 }
 
+// The same product for many positions. An item of k_ne_mfma decodes its weights
+// for 32 positions only, and reads x_hat from LDS once a wave and 32 rows: for
+// hundreds of positions the table lookups and those reads bound it. Here a
+// block of eight waves takes 64 RB rows x 128 positions and stages of 64
+// columns: every thread decodes RB runs of eight weights into LDS, once for the
+// 128 positions, and copies 64 bytes of x_hat; the waves, two by four, then
+// multiply 32 RB rows by 32 positions from LDS. A stage is decoded and stored
+// while the one before it is multiplied (two buffers, one barrier a stage), and
+// its words and x_hat are loaded a stage earlier still. A and B lie in LDS as
+// 64-lane fragments of 16-byte pieces, rows XORed so that stores and reads
+// spread over the banks.
+//
+// Bound by LDS: at 8192 x 2048 and 512 positions its accesses take 52% and the
+// matrix instructions 40% of the waves' 34 us (46 us a launch; k_ne_mfma 60),
+// about a quarter of the launch is the start and the write-back of Z. Stages
+// loaded one instead of two ahead: 49 us; half the waves multiplying while the
+// others decode: 48.
+constexpr uint32_t kWidePositions = 128;
+
+template <uint32_t RB>
+__global__ __launch_bounds__(kNeThreads) void k_ne_wide(NeMfmaJobs J) {
+    constexpr uint32_t kTileRows = 4u * RB;  // a block's
+    constexpr uint32_t kAPieces = 2u * RB * 4u * 64u, kBPieces = 4u * 4u * 2u * 64u;
+    __shared__ uint32_t table[1024];
+    __shared__ u32x4 a_lds[2][kAPieces];
+    __shared__ u32x4 b_lds[2][kBPieces];
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    // item (row group, K slice, position group, entry), fastest first
+    uint32_t rest = blockIdx.x;
+    const uint32_t rg = rest % J.row_groups;
+    rest /= J.row_groups;
+    const uint32_t ks = rest % J.k_slices;
+    rest /= J.k_slices;
+    const uint32_t pg = rest % J.position_groups;
+    const uint32_t which = rest / J.position_groups;
+    const NeMfma &a = J.ne[which];
+    const uint32_t stages = (a.columns >> 6) / J.k_slices;
+    const uint32_t p0 = pg * kWidePositions;
+    const uint2 tv = reinterpret_cast<const uint2 *>(J.ne_book)[t];
+    // run i of the thread: dword t % 32 (row (t % 32) / 2, columns 8 (t % 2) ..)
+    // of the tile in tile column (t / 32) % 4 and tile row t / 128 + 4 i; its
+    // second dword wraps within the tile (src/ne_trellis.hpp:196-200)
+    const uint32_t dword = t & 31u, tc = (t >> 5) & 3u;
+    const __amdgpu_buffer_rsrc_t wsrc = buffer_over(a.trellis, (a.tile_rows << a.tc_shift) * 128u);
+    uint32_t w_off[RB], a_slot[RB];
+#pragma unroll
+    for (uint32_t i = 0; i < RB; ++i) {
+        const uint32_t tr = (t >> 7) + 4u * i;
+        const uint32_t row = ((tr & 1u) << 4) | (dword >> 1), kh = dword & 1u;
+        w_off[i] = ((min(rg * kTileRows + tr, a.tile_rows - 1u) << a.tc_shift) + tc) * 128u;
+        a_slot[i] = ((tr >> 1) * 4u + tc) * 64u + kh * 32u + (row ^ (kh << 2));
+    }
+    // x_hat: 16 bytes (piece t % 8 of the stage's 128) of positions t / 8 and
+    // t / 8 + 64, both planes; positions past the batch repeat p0
+    const uint32_t piece = t & 7u;
+    const uint32_t x_bytes = a.batch * a.columns * 2u;
+    const __amdgpu_buffer_rsrc_t hi_src = buffer_over(a.x_hi, x_bytes), lo_src = buffer_over(a.x_lo, x_bytes);
+    uint32_t x_off[2], b_slot[2];
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+        const uint32_t pos = (t >> 3) + 64u * i;
+        x_off[i] = ((p0 + pos < a.batch ? p0 + pos : p0) * a.columns + 8u * piece) * 2u;
+        b_slot[i] = ((pos >> 5) * 4u + (piece >> 1)) * 128u + (piece & 1u) * 32u + ((pos & 31u) ^ piece);
+    }
+    struct Stage {
+        uint32_t d0[RB], d1[RB];
+        u32x4 hi[2], lo[2];
+    };
+    const auto load_stage = [&](uint32_t stage) {
+        Stage out;
+        const uint32_t at = ks * stages + stage;
+#pragma unroll
+        for (uint32_t i = 0; i < RB; ++i) {
+            out.d0[i] = __builtin_amdgcn_raw_buffer_load_b32(wsrc, w_off[i] + dword * 4u, at * 512u, 0);
+            out.d1[i] = __builtin_amdgcn_raw_buffer_load_b32(wsrc, w_off[i] + ((dword + 1u) & 31u) * 4u, at * 512u, 0);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+            out.hi[i] = __builtin_amdgcn_raw_buffer_load_b128(hi_src, x_off[i], at * 128u, 0);
+            out.lo[i] = __builtin_amdgcn_raw_buffer_load_b128(lo_src, x_off[i], at * 128u, 0);
+        }
+        return out;
+    };
+    const auto store_stage = [&](const Stage &s, uint32_t buffer) {
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+            b_lds[buffer][b_slot[i]] = s.hi[i];
+            b_lds[buffer][b_slot[i] + 64u] = s.lo[i];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < RB; ++i) {
+            u32x4 v;
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                v[q] = table[(state_hash_low16(window64(s.d0[i], s.d1[i], 8u * q)) >> 6) & 0x3FFu];
+            }
+            a_lds[buffer][a_slot[i]] = v;
+        }
+    };
+    const uint32_t m = lane & 31u, kh = lane >> 5;
+    const uint32_t wave_rows = wave & 1u, wave_positions = wave >> 1;
+    f32x16 acc[RB];
+#pragma unroll
+    for (uint32_t rb = 0; rb < RB; ++rb) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            acc[rb][r] = 0.0f;
+        }
+    }
+    struct Fragments {
+        half8 hi, lo, a[RB];
+    };
+    const auto read = [&](uint32_t buffer, uint32_t c) {
+        Fragments out;
+        const u32x4 *b = b_lds[buffer] + (wave_positions * 4u + c) * 128u + kh * 32u + (m ^ (2u * c + kh));
+        out.hi = __builtin_bit_cast(half8, b[0]);
+        out.lo = __builtin_bit_cast(half8, b[64]);
+#pragma unroll
+        for (uint32_t rb = 0; rb < RB; ++rb) {
+            out.a[rb] = __builtin_bit_cast(
+                half8, a_lds[buffer][((wave_rows * RB + rb) * 4u + c) * 64u + kh * 32u + (m ^ (kh << 2))]);
+        }
+        return out;
+    };
+    const auto multiply = [&](uint32_t buffer) {
+        Fragments f = read(buffer, 0);
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            Fragments ahead = f;
+            if (c < 3u) {
+                ahead = read(buffer, c + 1u);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t rb = 0; rb < RB; ++rb) {
+                acc[rb] = mfma32(f.a[rb], f.hi, acc[rb]);
+            }
+#pragma unroll
+            for (uint32_t rb = 0; rb < RB; ++rb) {
+                acc[rb] = mfma32(f.a[rb], f.lo, acc[rb]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            f = ahead;
+        }
+    };
+    // the words and x_hat of stage s wait in ring[s % 2]; loads past the last
+    // stage repeat it, unused
+    const uint32_t last = stages - 1u;
+    Stage ring[2] = {load_stage(0), load_stage(min(1u, last))};
+    table[2u * t] = tv.x;
+    table[2u * t + 1u] = tv.y;
+    __syncthreads();
+    store_stage(ring[0], 0);
+    ring[0] = load_stage(min(2u, last));
+    __syncthreads();
+    const auto step = [&](uint32_t stage, Stage &from) {  // `from` holds the stage after
+        store_stage(from, (stage + 1u) & 1u);
+        __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the products
+        from = load_stage(min(stage + 3u, last));
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(stage & 1u);
+        __syncthreads();
+    };
+    for (uint32_t stage = 0; stage + 2u < stages; stage += 2u) {
+        step(stage, ring[1]);
+        step(stage + 1u, ring[0]);
+    }
+    if (stages > 1u) {  // stages is a power of two
+        step(stages - 2u, ring[1]);
+    }
+    multiply(last & 1u);
+    // D register r of lane l: position l % 32, row (r % 4) + 8 (r / 4) + 4 kh
+    // of the 32-row block
+    const uint32_t p = p0 + 32u * wave_positions + m;
+    if (p < a.batch) {
+        float *z = a.z + static_cast<size_t>(ks) * a.batch * a.rows + static_cast<size_t>(p) * a.rows;
+#pragma unroll
+        for (uint32_t rb = 0; rb < RB; ++rb) {
+#pragma unroll
+            for (uint32_t g = 0; g < 4; ++g) {
+                const uint32_t row =
+                    (rg * kTileRows + 2u * (wave_rows * RB + rb)) * kTile + 8u * g + 4u * kh;
+                if (row < a.rows) {
+                    *reinterpret_cast<f32x4 *>(z + row) =
+                        f32x4{acc[rb][4 * g], acc[rb][4 * g + 1], acc[rb][4 * g + 2], acc[rb][4 * g + 3]} *
+                        a.weight_scale;
+                }
+            }
+        }
+    }
+}
+
+// Whether k_ne_wide takes a product: whole stages in every K slice, and at most
+// an eighth of its positions padding more than k_ne_mfma's, about what it gains
+// (8192 x 2048: 64 positions 16.1 us and 17.3, 128 23.0 and 19.1, 512 60 and 46).
+bool wide_takes(uint32_t columns, uint32_t batch, uint32_t k_slices) {
+    const uint32_t narrow = ceil_div(batch, 32u) * 32u, wide = ceil_div(batch, kWidePositions) * kWidePositions;
+    return columns / 64u >= k_slices && 8u * narrow >= 7u * wide;
+}
+
 }  // namespace
 
 uint32_t ne_mfma_slices(uint32_t rows, uint32_t columns, uint32_t batch) {
@@ -1017,8 +1218,18 @@ void launch_ne_mfma(adi_hip_context *ctx, NeMfmaJobs &J) {
     J.row_groups = ceil_div(n.rows / kTile, kNeItemTileRows);
     J.position_groups = ceil_div(n.batch, 32u);
     J.k_slices = ne_mfma_slices(n.rows, n.columns, n.batch);
+    auto kernel = k_ne_mfma;
+    if (wide_takes(n.columns, n.batch, J.k_slices)) {
+        // two row blocks a wave where one would take more than one block a CU
+        // (8192 x 2048, 512 positions: 46 us against 58; 4096 rows: 40, 31)
+        J.position_groups = ceil_div(n.batch, kWidePositions);
+        J.row_groups = ceil_div(n.rows, 64u);
+        const bool two = J.ne_count * J.position_groups * J.row_groups * J.k_slices > static_cast<uint32_t>(ctx->cu_count);
+        J.row_groups = two ? ceil_div(n.rows, 128u) : J.row_groups;
+        kernel = two ? k_ne_wide<2> : k_ne_wide<1>;
+    }
     J.items = J.ne_count * J.position_groups * J.row_groups * J.k_slices;
-    launch(ctx, "ne_mfma", k_ne_mfma, dim3(J.items), dim3(kNeThreads), 0, J);
+    launch(ctx, "ne_mfma", kernel, dim3(J.items), dim3(kNeThreads), 0, J);
 }
 
 }  // namespace adi_hip

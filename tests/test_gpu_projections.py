@@ -119,6 +119,27 @@ def test_ne_matmul_mfma(gpu, books, oracle, rows, columns, batch):
     assert max_rel_error(out.cpu().numpy(), want) <= MFMA_TOL
 
 
+@pytest.mark.parametrize("rows,columns,batch", [
+    (16, 64, 97), (16, 64, 96), (64, 128, 128), (128, 256, 129), (512, 2048, 193), (32, 4096, 127),
+    (2048, 128, 256), (8192, 64, 200), (8192, 64, 330), (8192, 128, 384), (4096, 32, 128)])
+def test_ne_matmul_wide(gpu, books, oracle, rows, columns, batch):
+    """Products of 97 positions and more, in blocks of 128 positions and 64 or
+    (8192 rows from 257 positions) 128 rows: one stage, several, K slices, rows and positions past
+    the matrix, and the sizes beside them that stay with 32 positions a block.
+    x_hat as f16 hi + lo holds 22 bits, so a sum of n random-sign terms stays
+    within sqrt(n) * 2^-22 <= 1.6e-5 of a term, under 1e-6 of the largest
+    output; 1e-5 leaves room for the float sums' order."""
+    _, nt, _, nb = books
+    rng = syn.rng_for(3, 7 * rows + columns + batch)
+    m = syn.ne_matrix(rng, rows, columns, nt)
+    x = syn.hidden_states(rng, batch, columns)
+    want = po.ne_matmul(oracle, m, x)
+    dm = hip.upload_ne(gpu, m, nb)
+    out = torch.empty((batch, rows), dtype=torch.float32, device="cuda")
+    hip.ne_matmul(gpu, dm, gpu.to_device(x), batch, out)
+    assert max_rel_error(out.cpu().numpy(), want) <= 1e-5
+
+
 @pytest.mark.parametrize("rows,columns", NE_SHAPES)
 @pytest.mark.parametrize("batch", [1, 3, 4, 7, 8, 16])
 def test_ne_matmul(gpu, books, oracle, rows, columns, batch):

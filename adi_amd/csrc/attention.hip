@@ -797,8 +797,8 @@ __global__ __launch_bounds__(256, 2) void k_attention_rows_one(const float *quer
 // (src/executor.cpp:480-496) and, for the query and key groups (blocks
 // 0-31), their L2 norm (497-505). The three inputs before token b are the
 // chunk's earlier qkv rows or, before the chunk, the state. With `shift` (one
-// token) the state shifts here; for a chunk k_conv_history does it after
-// every token has read it.
+// token) the state shifts here; for a chunk k_linear_norm_gate
+// does it, after every token has read it.
 __device__ __forceinline__ void linear_conv_token(const float *qkv, const uint16_t *weights,
                                                   float *state, float *convolved, uint32_t b,
                                                   bool shift) {
@@ -852,14 +852,9 @@ __global__ __launch_bounds__(kLinearHead) void k_linear_conv_rows(const float *q
                       convolved + static_cast<size_t>(r) * kChannels, 0, true);
 }
 
-// The convolution state after a chunk of `count` tokens: the last three of
-// (state, qkv rows) per channel.
-__global__ __launch_bounds__(256) void k_conv_history(const float *qkv, uint32_t count,
-                                                      float *state) {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= kChannels) {
-        return;
-    }
+// The convolution state of channel c after a chunk of `count` tokens: the last
+// three of (state, qkv rows).
+__device__ __forceinline__ void shift_history(const float *qkv, uint32_t count, float *state, uint32_t c) {
     float *history = state + static_cast<size_t>(c) * 3u;
     float next[3];
 #pragma unroll
@@ -1318,8 +1313,15 @@ __global__ __launch_bounds__(256) void k_linear_core_rows(const float *qkv, cons
 __global__ __launch_bounds__(kLinearHead) void k_linear_norm_gate(const float *recurrent_output,
                                                                   const uint16_t *norm,
                                                                   const float *gate,
-                                                                  float *normalized) {
+                                                                  float *normalized, const float *qkv,
+                                                                  float *convolution) {
 #pragma clang fp contract(off)
+    if (blockIdx.x == kValueHeads) {  // the grid's last column, after a chunk: the convolution state
+        for (uint32_t c = blockIdx.y * kLinearHead + threadIdx.x; c < kChannels; c += gridDim.y * kLinearHead) {
+            shift_history(qkv, gridDim.y, convolution, c);
+        }
+        return;
+    }
     __shared__ float partial[16];
     const size_t i = static_cast<size_t>(blockIdx.y) * kValueSize +
                      static_cast<size_t>(blockIdx.x) * kLinearHead + threadIdx.x;
@@ -1585,10 +1587,6 @@ void linear_attention_chunk(adi_hip_context *ctx, const adi_hip_linear_attention
     launch(ctx, "linear_conv", k_linear_conv, dim3(kChannels / kLinearHead, count),
            dim3(kLinearHead), 0, static_cast<const float *>(qkv), L->convolution,
            convolution_state, convolved);
-    if (count > 1) {
-        launch(ctx, "linear_conv_history", k_conv_history, dim3(kChannels / 256), dim3(256), 0,
-               static_cast<const float *>(qkv), count, convolution_state);
-    }
     const dim3 delta_grid(kValueHeads, kLinearHead / kDeltaRows);
     if (count == 1) {  // the decode step's bits
         LinearRows table{};
@@ -1606,9 +1604,11 @@ void linear_attention_chunk(adi_hip_context *ctx, const adi_hip_linear_attention
                static_cast<const float *>(beta + static_cast<size_t>(b0) * kValueHeads), L->alpha_bias, L->a_log,
                n, recurrent_state, recurrent_output + static_cast<size_t>(b0) * kValueSize);
     }
-    launch(ctx, "linear_norm_gate", k_linear_norm_gate, dim3(kValueHeads, count),
+    // a chunk's state shifts here, where every token has read it, in blocks of
+    // its own (a launch for it alone took 4.7 us)
+    launch(ctx, "linear_norm_gate", k_linear_norm_gate, dim3(count > 1 ? kValueHeads + 1 : kValueHeads, count),
            dim3(kLinearHead), 0, static_cast<const float *>(recurrent_output), L->norm,
-           static_cast<const float *>(gate), normalized);
+           static_cast<const float *>(gate), normalized, static_cast<const float *>(qkv), convolution_state);
     project_output(ctx, &L->output, normalized, count, outputs, norm_tail);
 }
 
@@ -1837,7 +1837,8 @@ void linear_attention_rows(adi_hip_context *ctx, const adi_hip_linear_attention 
                recurrent_output + at * kValueSize);
         launch(ctx, "linear_norm_gate", k_linear_norm_gate, dim3(kValueHeads, count), dim3(kLinearHead),
                0, static_cast<const float *>(recurrent_output + at * kValueSize), L->norm,
-               static_cast<const float *>(gate + at * kValueSize), normalized + at * kValueSize);
+               static_cast<const float *>(gate + at * kValueSize), normalized + at * kValueSize,
+               static_cast<const float *>(nullptr), static_cast<float *>(nullptr));
     }
     project_output(ctx, &L->output, normalized, rows, outputs, norm_tail);
 }

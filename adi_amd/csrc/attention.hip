@@ -579,22 +579,21 @@ __global__ __launch_bounds__(256, 2) void k_attention_partial_rows(const float *
 // The splits of one query head merged (splits <= N): every split's
 // accumulator, then the splits' maxima and denominators (through LDS),
 // loaded in one round, then the accumulators added in split order.
-template <uint32_t N, bool COHERENT = false>
+template <uint32_t N>
 __device__ __forceinline__ void combine_splits(const float *p, uint32_t splits, uint32_t t, float *split_max,
                                                float *split_den, float *split_factor, float &a, float &d) {
 #pragma clang fp contract(off)
-    const auto load = [](const float *at) { return COHERENT ? coherent_load(at) : *at; };
     float acc[N];
 #pragma unroll
     for (uint32_t s = 0; s < N; ++s) {
-        acc[s] = s < splits ? load(p + s * kPartialStride + t) : 0.0f;
+        acc[s] = s < splits ? p[s * kPartialStride + t] : 0.0f;
     }
     static_assert(N <= kHeadSize, "a thread's split");
     // both words of the thread's split loaded before either is stored (one
     // round trip with the accumulators')
     if (t < splits) {
-        const float mx = load(p + t * kPartialStride + kHeadSize);
-        const float dn = load(p + t * kPartialStride + kHeadSize + 1);
+        const float mx = p[t * kPartialStride + kHeadSize];
+        const float dn = p[t * kPartialStride + kHeadSize + 1];
         split_max[t] = mx;
         split_den[t] = dn;
     }

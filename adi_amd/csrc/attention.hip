@@ -20,10 +20,12 @@
 //   A long chunk's partial runs on the matrix cores (attention_chunk.hip).
 // Linear attention, after the projections:
 //   conv        per 128-channel group: the width-4 causal convolution, SiLU,
-//               the state shift, and the L2 norm of the query and key heads
+//               one token's state shift, and the L2 norm of the query and key
+//               heads
 //   delta       block (value head, 16 rows): the gated delta update of each
-//               state row, one wave per row, state read and written once
-//   norm_gate   per value head: RMS norm (weight offset 0) times SiLU(gate)
+//               state row, state read and written once
+//   norm_gate   per value head: RMS norm (weight offset 0) times SiLU(gate);
+//               after a chunk also the convolution's state shift
 // The sums run in a different order from the CPU's (wave and block
 // reductions); results agree to float rounding.
 #include "attention.hpp"

@@ -288,6 +288,12 @@ __device__ __forceinline__ uint32_t descending_key(float v) {
     return ~ascending;
 }
 
+// The logit of a key.
+__device__ __forceinline__ float logit_of_key(uint32_t key) {
+    const uint32_t ascending = ~key;
+    return __uint_as_float((ascending & 0x80000000u) != 0u ? ascending ^ 0x80000000u : ~ascending);
+}
+
 // a / t, correctly rounded, from t's correctly rounded reciprocal: the first
 // product is within an ulp, and its exact remainder corrects it (Markstein).
 __device__ __forceinline__ double quotient(double a, double t, double inverse) {
@@ -300,14 +306,17 @@ __device__ __forceinline__ double quotient(double a, double t, double inverse) {
 // exp((v - max) / t) in double over span p, each thread in index order, then
 // a fixed tree; k_sample_rows adds the spans' sums in span order. A row with
 // a non-finite logit (a span index of 0xFFFFFFFF) gets sums of 0: the
-// sampler rejects it. The bins take only tokens that can matter: those below
-// p = (1 - top_p) / (1000 count) hold together less than a thousandth of what
-// top_p leaves out, and an LDS atomic on one of the few bins of a normal tail
-// waits for its neighbours' (16 rows of 248,320 logits, temperature 0.7, top_p
-// 0.9: 36 us with every token binned, 25 us).
+// sampler rejects it. Only bins that can matter take their tokens, every one of
+// them: tokens below p = (1 - top_p) / (1000 count) hold together less than a
+// thousandth of what top_p leaves out, so the bins behind the one of that p's
+// logit stay empty. An LDS atomic on one of the few bins of a normal tail waits
+// for its neighbours' (16 rows of 248,320 logits, temperature 0.7, top_p 0.9:
+// 36 us with every token binned, 25 us). A bin is taken whole because a bin is
+// an eighth of a binade of the logit and at a low temperature or a large logit
+// holds tokens of both kinds; the walks count a bin's tokens by these counts.
 __global__ __launch_bounds__(kArgmaxPartThreads) void k_expsum_parts(
     const float *logits, uint32_t count, uint32_t span, const float *part_value,
-    const uint32_t *part_index, float temperature, float top_p, double *part_sum, uint32_t *top) {
+    const uint32_t *part_index, float temperature, double reach, double *part_sum, uint32_t *top) {
     __shared__ double wave_sum[kArgmaxPartThreads / kWave];
     // with `top`: the span's bin counts and masses, added into the row's
     __shared__ uint32_t bin_count[kTopBins];
@@ -339,12 +348,14 @@ __global__ __launch_bounds__(kArgmaxPartThreads) void k_expsum_parts(
         __syncthreads();
     }
     double part = 0.0;
-    const double negligible = (1.0 - static_cast<double>(top_p)) * 1e-3 / static_cast<double>(count);
+    // the smallest logit of the bin of that p's logit, maximum + reach
+    const double least = fmax(maximum + reach, -static_cast<double>(__FLT_MAX__));
+    const float edge = logit_of_key(descending_key(static_cast<float>(least)) | ((1u << kTopShift) - 1u));
     const double inverse = 1.0 / t;
     for_each_logit(row, end - begin, [&](uint32_t, float v) {
         const double p = exp(quotient(static_cast<double>(v) - maximum, t, inverse));
         part += p;
-        if (top != nullptr && p >= negligible) {
+        if (top != nullptr && v >= edge) {
             const uint32_t bin = descending_key(v) >> kTopShift;
             atomicAdd(&bin_count[bin], 1u);
             atomicAdd(&bin_mass[bin], static_cast<float>(p));
@@ -1081,9 +1092,9 @@ __global__ __launch_bounds__(kSampleThreads) void k_sample_rows(const float *log
 // bin whose inclusive mass reaches top_p of the row's sum, by a 0.1% margin
 // over the bins' float masses, when it holds at most kWindow tokens. Every
 // block (p, r) finds the same cut from the row's bins and appends its span's
-// tokens before it; block (0, r) records how many the prefix holds. A row
-// with a non-finite logit, or whose cut is out of reach, is left to the
-// full sampler.
+// tokens up to it; block (0, r) records how many the prefix holds by the bins'
+// counts, which k_top_walk compares with how many were appended. A row with a
+// non-finite logit, or whose cut is out of reach, is left to the full sampler.
 __global__ __launch_bounds__(kArgmaxPartThreads) void k_top_collect(const float *logits, uint32_t count,
                                                                     uint32_t span, const uint32_t *part_index,
                                                                     const double *part_sum, float top_p,
@@ -1184,7 +1195,9 @@ __global__ __launch_bounds__(kArgmaxPartThreads) void k_top_collect(const float 
                 at = atomicAdd(&words[kTopState], static_cast<uint32_t>(__popcll(kept)));
             }
             at = static_cast<uint32_t>(__shfl(static_cast<int>(at), leader)) + before;
-            cand[at] = (static_cast<uint64_t>(key) << 32) | (begin + i);
+            if (at < kWindow) {
+                cand[at] = (static_cast<uint64_t>(key) << 32) | (begin + i);
+            }
         }
     });
 }
@@ -1202,8 +1215,9 @@ __global__ __launch_bounds__(kArgmaxPartThreads) void k_top_walk(const float *lo
     __shared__ uint64_t cand[kWindow];
     __shared__ double prob[kWindow], share[kWindow];
     uint32_t *state = top + static_cast<size_t>(blockIdx.x) * kTopRowWords;
-    const uint32_t n = state[kTopState + 1];
-    if (n == 0u) {
+    const uint2 counts = *reinterpret_cast<const uint2 *>(state + kTopState);
+    const uint32_t n = counts.y;
+    if (n == 0u || counts.x != n) {  // no prefix, or not all of it and nothing else
         return;
     }
     const float *row = logits + static_cast<size_t>(blockIdx.x) * count;
@@ -1329,9 +1343,13 @@ int adi_hip_sample_rows(adi_hip_context *ctx, const float *logits, uint32_t rows
         uint32_t *top = ws.take<uint32_t>(size_t(rows) * kTopRowWords);
         launch(ctx, "argmax_parts", k_argmax_parts, dim3(parts, rows), dim3(kArgmaxPartThreads), 0,
                logits, count, span, part_value, part_index, top, kTopZeroWords, kTopRowWords);
+        // the log of the p below which a token cannot matter (top_p 1: -inf),
+        // as a distance from the row's maximum
+        const double reach = static_cast<double>(temperature) *
+                             std::log((1.0 - static_cast<double>(top_p)) * 1e-3 / static_cast<double>(count));
         launch(ctx, "expsum_parts", k_expsum_parts, dim3(parts, rows), dim3(kArgmaxPartThreads), 0,
                logits, count, span, static_cast<const float *>(part_value),
-               static_cast<const uint32_t *>(part_index), temperature, top_p, part_sum, top);
+               static_cast<const uint32_t *>(part_index), temperature, reach, part_sum, top);
         // the short walk: the kept set of most rows ends in a short prefix of
         // the sorted order; the full sampler then only runs for the rest
         launch(ctx, "top_collect", k_top_collect, dim3(parts, rows), dim3(kArgmaxPartThreads), 0, logits,

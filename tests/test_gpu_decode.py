@@ -171,6 +171,48 @@ def test_sample_rows_wide_kept_sets(gpu, oracle, temperature, top_p):
     assert got.tolist() == want
 
 
+def straddling_rows(rng, count, temperature):
+    """Rows whose likely tokens share a bin of the sampler (an eighth of a
+    binade of the logit) with tokens too unlikely to matter, at the edges of
+    what the short walk takes."""
+    if temperature == 0.05:
+        # four tokens in one bin, the first of them negligible
+        three = rng.normal(0, 0.5, count)
+        three[[5, 100, 200, 300]] = 16.2, 17.9, 17.9 + 0.05 * np.log(0.55), 17.9 + 0.05 * np.log(0.30)
+        rows = [three, rng.normal(0, 8, count), rng.normal(6, 0.3, count), rng.normal(-140, 0.5, count)]
+    elif temperature == 0.2:
+        far, below = rng.normal(97, 0.5, count), rng.normal(-140, 0.5, count)
+        far[7], below[9] = 103.9, -130.0
+        rows = [rng.normal(100, 2, count), far, below, rng.normal(0, 3, count)]
+    elif temperature == 0.4:
+        rows = [rng.normal(260, 2, count) for _ in range(3)] + [rng.normal(-20, 0.5, count)]
+        rows[0][rng.integers(0, count, 16)] += 12.0
+        rows[1][count - 1] += 30.0
+    else:
+        close = rng.normal(5.05, 0.01, count)
+        close[[0, 9, 99, 999, 9999]] = 5.4
+        rows = [close, rng.uniform(-1, 1, count), rng.normal(60, 2, count), rng.normal(0, 2, count)]
+    return np.stack(rows).astype(np.float32)
+
+
+@pytest.mark.parametrize("temperature,top_p", [(1e-4, 0.9), (1e-3, 0.8), (0.01, 0.9), (0.02, 0.9), (0.05, 0.7),
+                                               (0.1, 0.9), (0.2, 0.9), (0.4, 0.9), (0.4, 0.05)])
+def test_sample_rows_bins_of_mixed_tokens(gpu, oracle, temperature, top_p):
+    """Low temperatures and large or offset logits, where one bin holds tokens
+    that can matter and tokens that cannot: the short walk's prefix is whole
+    bins, so it holds the tokens that its count says, and a prefix longer than
+    its room leaves the row, and the rows beside it, to the other walks. Each
+    row takes three draws."""
+    rng = np.random.default_rng(int(temperature * 10000 + top_p * 100))
+    base = straddling_rows(rng, 248320, temperature)
+    logits = np.concatenate([base, base[::-1], base])
+    words = rng.integers(0, 2**63, len(logits), dtype=np.uint64) * 2
+    words[0] = 2**64 - 1
+    got = sample_device(gpu, logits, temperature, top_p, words)
+    want = [po.sample_token(oracle, logits[r], temperature, top_p, int(words[r])) for r in range(len(logits))]
+    assert got.tolist() == want
+
+
 def test_sample_rows_small_vocabularies_and_edges(gpu, oracle):
     rng = np.random.default_rng(77)
     for count in (1, 2, 63, 4096, 4097, 12289):

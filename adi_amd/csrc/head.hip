@@ -678,7 +678,12 @@ __global__ __launch_bounds__(kHmThreads) void k_head_mfma_many(const uint8_t *__
     const uint32_t tiles = (rows + kHmTile - 1u) / kHmTile;
     const uint32_t q = lane / 16u, n = lane % 16u;
     const uint32_t shift = 16u * (q & 1u);
-    // loads past the last row give zeros
+    // A tile's first row: a tile that reaches past the last row, and one past
+    // the last tile, takes the last 16 rows instead, so that every load lies
+    // inside the codes and scales (a buffer's range check leaves the scalar
+    // offset out). With fewer than 16 rows the last one stands for the rest.
+    const uint32_t last_start = rows > kHmTile ? rows - kHmTile : 0u, last_row = min(rows, kHmTile) - 1u;
+    const auto row_of_tile = [&](uint32_t tile) { return min(tile * kHmTile, last_start); };
     const __amdgpu_buffer_rsrc_t code_buffer =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(packed), 0, rows * 1280u, 0x00020000);
     const __amdgpu_buffer_rsrc_t scale_buffer =
@@ -692,25 +697,27 @@ __global__ __launch_bounds__(kHmThreads) void k_head_mfma_many(const uint8_t *__
 #pragma unroll
     for (uint32_t k = 0; k < kHmRawLoads; ++k) {
         const uint32_t e = 64u * k + lane;
-        code_from[k] = e / 20u * 1280u + 16u * (e % 20u);
+        code_from[k] = min(e / 20u, last_row) * 1280u + 16u * (e % 20u);
         code_to[k] = (e / 20u * kHmStagePitch + 16u * (e % 20u)) / 4u;
     }
-    const uint32_t scale_from = (lane & 31u) * 64u;
+    const uint32_t scale_from = min(lane & 15u, last_row) * 64u;
     // quarter kq of the codes and scales (lanes 0-31: a row's 8 groups) of
     // `count` tiles
     const auto load = [&]<uint32_t COUNT>(std::integral_constant<uint32_t, COUNT>, uint32_t tile0, uint32_t kq,
                                           Raw &out) {
 #pragma unroll
         for (uint32_t tile = 0; tile < COUNT; ++tile) {
-            const uint32_t at = (tile0 + tile) * kHmTile * 1280u + kHmPieceBytes * kq;
+            const uint32_t at = row_of_tile(tile0 + tile) * 1280u + kHmPieceBytes * kq;
 #pragma unroll
             for (uint32_t k = 0; k < kHmRawLoads; ++k) {
                 out.codes[tile][k] = __builtin_bit_cast(
                     hm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(code_buffer, code_from[k], at, 0));
             }
         }
-        out.scales = __builtin_bit_cast(hm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                      scale_buffer, scale_from, tile0 * kHmTile * 64u + 16u * kq, 0));
+        const uint32_t row0 = row_of_tile(tile0), row1 = row_of_tile(tile0 + 1u);
+        out.scales = __builtin_bit_cast(
+            hm_u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                          scale_buffer, scale_from + ((lane & 16u) != 0u ? row1 - row0 : 0u) * 64u, row0 * 64u + 16u * kq, 0));
     };
     using One = std::integral_constant<uint32_t, 1>;
     using Two = std::integral_constant<uint32_t, 2>;
@@ -785,8 +792,8 @@ __global__ __launch_bounds__(kHmThreads) void k_head_mfma_many(const uint8_t *__
                 }
             }
             __syncthreads();
-            // (the one column past 3 batch of a last table holds old values,
-            // or none yet; nothing reads its sums)
+            // (columns of tokens past the batch are zeros; nothing reads their
+            // sums)
             if (threadIdx.x < TABLES * kHmChunk * 16u) {
                 const float *part = &L.u.part[0][0][0][0] + 8u * threadIdx.x;
                 float k = 0.0f;
@@ -886,13 +893,15 @@ __global__ __launch_bounds__(kHmThreads) void k_head_mfma_many(const uint8_t *__
                 }
                 fence();
                 const uint32_t t = lane / 4u, row = 4u * (lane % 4u);
-                const uint32_t global = (tile_of(r) + tile) * kHmTile + row;
+                const uint32_t at = (tile_of(r) + tile) * kHmTile;
+                const uint32_t global = row_of_tile(tile_of(r) + tile) + row;
                 if (t < batch) {
                     float *to = logits + static_cast<size_t>(t) * rows + global;
 #pragma unroll
                     for (uint32_t j = 0; j < 4; ++j) {
                         const float *piece = &L.u.sums[wave][row + j][3u * t];
-                        if (global + j < rows) {
+                        // (the rows before `at` are the tile before's)
+                        if (global + j >= at && global + j < rows) {
                             to[j] = (piece[0] + piece[1]) + piece[2];
                         }
                     }

@@ -1320,6 +1320,22 @@ bool head_wave_best(const adi_hip_head_chunk *h) {
     return h->columns == 2048u && h->protected_count == 0;
 }
 
+// Whether one pass for `tokens` (at most sixteen) beats passes of four. Where
+// k_head_mfma's waves have several tiles each, from five tokens on (40,960 rows,
+// 5, 8, 12, 16 tokens: 39, 40, 56, 74 us in passes, 27, 34, 39, 43 in one). Where
+// each has one tile at most, a pass of four is little more than its tables, and
+// one pass builds four times as many quarters of them: 2,048 rows 5, 8, 9, 12,
+// 16 tokens take 22.7, 23.1, 32.3, 32.8, 42.7 us in passes, 24.4, 30.3, 31.0,
+// 35.8, 39.6 in one; 32,768 rows 28.9, 29.4, 40.7, 41.5, 53.5 and 26.6, 32.5,
+// 33.4, 38.3, 42.3.
+bool head_many_takes(const adi_hip_context *ctx, uint32_t rows, uint32_t tokens) {
+    const uint32_t passes = ceil_div(tokens, kHmTokens), tables = ceil_div(3u * tokens, 16);
+    if (ceil_div(rows, kHmTile) > static_cast<uint32_t>(ctx->cu_count) * kHmWaves) {
+        return passes > 1u;
+    }
+    return passes > 2u && tables < passes;
+}
+
 // Logits of five to sixteen tokens (16-byte aligned codes).
 void launch_head_many(adi_hip_context *ctx, const adi_hip_head_chunk *h, const float *x, uint32_t batch,
                       float *logits) {
@@ -1372,12 +1388,15 @@ void head_logits(adi_hip_context *ctx, const adi_hip_head_chunk *h, const float 
                 set_lds_limit(reinterpret_cast<const void *>(&k_head_mfma<true, false>), sizeof(HeadMfmaLds)) &&
                 set_lds_limit(reinterpret_cast<const void *>(&k_head_mfma<false, false>), sizeof(HeadMfmaLds));
             (void)ready;
-            // without bounds, five tokens and more go sixteen at a time through
-            // one pass over the codes, what is left (up to four) as before
+            // without bounds, tokens go sixteen at a time through one pass over
+            // the codes, those that take it no faster in passes of four
             uint32_t t0 = 0;
             const bool addressed = size_t(h->rows) + 64u <= 0xFFFFFFFFu / 1280u;  // by 32-bit offsets
-            while (bounds == nullptr && coalesced && addressed && batch - t0 > kHmTokens) {
+            while (bounds == nullptr && coalesced && addressed && t0 < batch) {
                 const uint32_t tokens = std::min(batch - t0, kHmManyTokens);
+                if (!head_many_takes(ctx, h->rows, tokens)) {
+                    break;
+                }
                 launch_head_many(ctx, h, x + size_t(t0) * 2048u, tokens, logits + size_t(t0) * h->rows);
                 t0 += tokens;
             }

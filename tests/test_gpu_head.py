@@ -60,7 +60,8 @@ def test_head_2048_columns_by_batch(gpu, oracle, batch):
 
 
 @pytest.mark.parametrize("rows,batches", [(1, [5, 16]), (7, [5, 16]), (15, [6]), (16, [5, 11]), (17, [7, 16]),
-                                          (31, [5]), (32, [16]), (33, [6, 17]),
+                                          (31, [5, 9]), (32, [10, 16]),
+                                          (33, [6, 17]), (32768, [5, 8, 9, 12]), (32769, [5, 6, 11]),
                                           (1000, [5, 6, 10, 11, 16, 21, 32, 37]), (4097, [8, 16]), (170001, [9]),
                                           (170016, [5])])
 def test_head_many_tokens_equal_single_tokens(gpu, rows, batches):
@@ -70,7 +71,8 @@ def test_head_many_tokens_equal_single_tokens(gpu, rows, batches):
     the five tiles that each wave holds at once. A tile that reaches past the
     last row is the last 16 rows, of which it stores its own; a wave without
     tiles reads those 16 too, and with fewer rows than 16 the last again. The
-    codes end where their allocation does."""
+    codes end where their allocation does. Up to 32,768 rows (a tile a wave on
+    256 CUs) 5 to 8, 11 and 12 tokens take passes of four."""
     rng = syn.rng_for(1, 6000 + rows)
     dh = hip.upload_head(gpu, syn.head_chunk(rng, rows, 2048, 0))
     x = gpu.to_device(syn.rms_normalized(syn.hidden_states(rng, max(batches), 2048)))

@@ -331,6 +331,16 @@ __device__ __forceinline__ void expert_small_slots(const ExpertMfmaJobs &J, uint
             }
         }
     };
+    // a unit's gamma rows: written by every lane as halves, read by others in
+    // fours
+    const auto store_gammas = [&](uint2 *to, uint32_t a, uint32_t b, uint32_t c) {
+        store_gamma(to, lane, a);
+        store_gamma(to, lane + 64u, b);
+        store_gamma(to, lane + 128u, c);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     struct Step {
         ExpertWords words;
         half8 hi, lo;
@@ -367,9 +377,7 @@ __device__ __forceinline__ void expert_small_slots(const ExpertMfmaJobs &J, uint
     }
     uint32_t load_kc = 4u;
     uint2 *gamma_now = gammas, *gamma_next = gammas + 4u * kSmallGammaRow;
-    store_gamma(gamma_now, lane, g0);
-    store_gamma(gamma_now, lane + 64u, g1);
-    store_gamma(gamma_now, lane + 128u, g2);
+    store_gammas(gamma_now, g0, g1, g2);
     SmallUnit now = load;
     bool more = false;  // `load` is past `now`
     uint32_t kc = 0;
@@ -440,9 +448,7 @@ __device__ __forceinline__ void expert_small_slots(const ExpertMfmaJobs &J, uint
             uint2 *const spent = gamma_now;
             gamma_now = gamma_next;
             gamma_next = spent;
-            store_gamma(gamma_now, lane, g0);
-            store_gamma(gamma_now, lane + 64u, g1);
-            store_gamma(gamma_now, lane + 128u, g2);
+            store_gammas(gamma_now, g0, g1, g2);
             now = load;
             kc = 0;
 #pragma unroll

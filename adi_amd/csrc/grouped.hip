@@ -993,12 +993,18 @@ __global__ __launch_bounds__(kNeThreads) void k_ne_wide(NeMfmaJobs J) {
     __shared__ u32x4 b_lds[2][kBPieces];
     const uint32_t t = threadIdx.x, lane = t & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    // item (row group, K slice, position group, entry), fastest first
-    uint32_t rest = blockIdx.x;
+    // item (row group, K slice, position group, entry), fastest first. With
+    // eight K slices or more the slices come first: block b runs on XCD b % 8,
+    // so an XCD then reads x_hat and weights of its slices only, where eight row
+    // groups first had every XCD read all of x_hat (512 x 2048, 256 positions:
+    // 20.0 us a call, 17.3; k_ne_mfma 18.3).
+    const bool by_slice = J.k_slices >= 8u;
+    const uint32_t slice_shift = __builtin_ctz(J.k_slices);  // (a power of two)
+    uint32_t rest = by_slice ? blockIdx.x >> slice_shift : blockIdx.x;
     const uint32_t rg = rest % J.row_groups;
     rest /= J.row_groups;
-    const uint32_t ks = rest % J.k_slices;
-    rest /= J.k_slices;
+    const uint32_t ks = (by_slice ? blockIdx.x : rest) & (J.k_slices - 1u);
+    rest = by_slice ? rest : rest >> slice_shift;
     const uint32_t pg = rest % J.position_groups;
     const uint32_t which = rest / J.position_groups;
     const NeMfma &a = J.ne[which];
@@ -1160,7 +1166,11 @@ __global__ __launch_bounds__(kNeThreads) void k_ne_wide(NeMfmaJobs J) {
 
 // Whether k_ne_wide takes a product: whole stages in every K slice, and at most
 // an eighth of its positions padding more than k_ne_mfma's, about what it gains
-// (8192 x 2048: 64 positions 16.1 us and 17.3, 128 23.0 and 19.1, 512 60 and 46).
+// (8192 x 2048: 64 positions 16.1 us and 17.3, 128 23.0 and 19.1, 512 60 and 46;
+// whole calls of 97, 128, 256 and 512 positions: 512 x 2048 15.4, 15.7, 18.3,
+// 20.6 us and 14.3, 14.8, 17.3, 19.3; 2048 x 512 14.3, 14.6, 17.2, 20.6 and
+// 13.3, 13.9, 16.5, 19.4; 2048 x 4096 23.0, 24.8, 29.9, 45.8 and 19.7, 21.3,
+// 27.4, 40.3).
 bool wide_takes(uint32_t columns, uint32_t batch, uint32_t k_slices) {
     const uint32_t narrow = ceil_div(batch, 32u) * 32u, wide = ceil_div(batch, kWidePositions) * kWidePositions;
     return columns / 64u >= k_slices && 8u * narrow >= 7u * wide;

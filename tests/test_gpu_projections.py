@@ -121,11 +121,12 @@ def test_ne_matmul_mfma(gpu, books, oracle, rows, columns, batch):
 
 @pytest.mark.parametrize("rows,columns,batch", [
     (16, 64, 97), (16, 64, 96), (64, 128, 128), (128, 256, 129), (512, 2048, 193), (32, 4096, 127),
-    (2048, 128, 256), (8192, 64, 200), (8192, 64, 330), (8192, 128, 384), (4096, 32, 128)])
+    (2048, 128, 256), (8192, 64, 200), (8192, 64, 330), (8192, 128, 384), (4096, 32, 128),
+    (512, 2048, 128), (512, 2048, 250), (512, 2048, 300), (2048, 4096, 97)])
 def test_ne_matmul_wide(gpu, books, oracle, rows, columns, batch):
     """Products of 97 positions and more, in blocks of 128 positions and 64 or
-    (8192 rows from 257 positions) 128 rows: one stage, several, K slices, rows and positions past
-    the matrix, and the sizes beside them that stay with 32 positions a block.
+    (8192 rows from 257 positions) 128 rows: one stage, several, K slices (eight and more of them
+    dealt before the row groups), rows and positions past the matrix, and the sizes beside them that stay with 32 positions a block.
     x_hat as f16 hi + lo holds 22 bits, so a sum of n random-sign terms stays
     within sqrt(n) * 2^-22 <= 1.6e-5 of a term, under 1e-6 of the largest
     output; 1e-5 leaves room for the float sums' order."""

@@ -30,10 +30,10 @@
 // vector kernel 3048 (each query head of each token read the history again).
 // Four waves of 32 rows with v_mfma_f32_32x32x16, one a SIMD: 200 us.
 //
-// A block that meets a value the pieces cannot stand for (an infinity, a NaN,
-// a query or key that rounds to an f16 infinity) starts over in plain floats,
-// entry by entry, a wave a row, as the vector kernel does: a row skips the
-// entries behind its position, which a matrix product multiplies by zero.
+// A tile with a value the pieces cannot stand for (an infinity, a NaN, a query
+// or key that rounds to an f16 infinity) runs in plain floats, entry by entry,
+// on the same running state: a row skips the entries behind its position, which
+// a matrix product multiplies by zero.
 #include "attention.hpp"
 
 namespace adi_hip {
@@ -145,44 +145,6 @@ __device__ __forceinline__ float weight_of(float d) {
     return fmaf(y * tail, kLn2, y);
 }
 
-// The wave's 16 rows (2 tokens from wave_token, 8 heads) over keys first ..
-// end - 1 in plain floats, one row after another, lane l dimensions 4 l ..
-// 4 l + 3.
-__device__ __forceinline__ void rows_in_floats(const ChunkArgs &args, uint32_t kv, uint32_t split, uint32_t wave_token,
-                                            uint32_t first, uint32_t end) {
-    const uint32_t lane = threadIdx.x & 63u;
-    for (uint32_t i = 0; i < kWaveTokens * kHeads && wave_token + i / kHeads < args.count; ++i) {
-        const uint32_t token = wave_token + i / kHeads, head = kv * kHeads + i % kHeads;
-        const size_t row = static_cast<size_t>(token) * kQueryHeads + head;
-        const float4 *query = reinterpret_cast<const float4 *>(args.query_gate + row * 2u * kHeadSize);
-        const float4 q = query[lane];
-        float maximum = -__builtin_huge_valf(), denominator = 0.0f;
-        float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (uint32_t key = first; key < min(end, args.position + token + 1u); ++key) {
-            const size_t at = (static_cast<size_t>(key) * kKvHeads + kv) * kHeadSize;
-            const float4 k = reinterpret_cast<const float4 *>(args.keys + at)[lane];
-            const float4 v = reinterpret_cast<const float4 *>(args.values + at)[lane];
-            const float dot = wave_sum(((q.x * k.x + q.y * k.y) + q.z * k.z) + q.w * k.w);
-            online_step(dot * 0.0625f, v, maximum, denominator, acc);
-        }
-        if (args.splits == 1u) {
-            const float inverse = 1.0f / denominator;
-            const float4 g = query[kHeadSize / 4u + lane];
-            reinterpret_cast<float4 *>(args.attended + row * kHeadSize)[lane] =
-                make_float4(acc.x * inverse * sigmoid_of(g.x), acc.y * inverse * sigmoid_of(g.y),
-                            acc.z * inverse * sigmoid_of(g.z), acc.w * inverse * sigmoid_of(g.w));
-            continue;
-        }
-        float *to = args.partial + (row * args.splits + split) * kPartialStride;
-        reinterpret_cast<float2 *>(to)[2u * lane] = make_float2(acc.x, acc.y);
-        reinterpret_cast<float2 *>(to)[2u * lane + 1u] = make_float2(acc.z, acc.w);
-        if (lane == 0) {
-            to[kHeadSize] = maximum;
-            to[kHeadSize + 1u] = denominator;
-        }
-    }
-}
-
 __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args) {
     extern __shared__ __align__(16) unsigned char lds[];
     unsigned char *const key_lds = lds;
@@ -221,21 +183,6 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
     if (t < 3u) {
         odd[t] = kNoTile;
     }
-    // the row's query in pieces: step s holds dimensions 32 s + 8 quarter +
-    // 0 .. 7
-    u32x4 q[8][kKeyPieces];
-    uint32_t big_query = 0;
-#pragma unroll
-    for (uint32_t s = 0; s < 8u; ++s) {
-        const float4 *from = reinterpret_cast<const float4 *>(query + 32u * s + 8u * quarter);
-        const float4 a = from[0], b = from[1];
-        big_query = largest(largest(big_query, a), b);
-        const HalfPieces c0 = split_pair_f16(a.x, a.y), c1 = split_pair_f16(a.z, a.w);
-        const HalfPieces c2 = split_pair_f16(b.x, b.y), c3 = split_pair_f16(b.z, b.w);
-        q[s][0] = u32x4{c0.hi, c1.hi, c2.hi, c3.hi};
-        q[s][1] = u32x4{c0.lo, c1.lo, c2.lo, c3.lo};
-    }
-
     // A tile's entries pass through registers, each wave four key rows and
     // four value rows (4 wave + 0 .. 3), lane l dimensions 4 l .. 4 l + 3.
     // Rows past the chunk's last entry repeat it (behind every row's
@@ -274,147 +221,244 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
         out[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
     float maximum = -__builtin_huge_valf(), denominator = 0.0f;
-    bool exact = true;  // every value so far has its pieces
 
-    if (tile0 < tile_end) {
+    // A tile in floats: its entries to LDS (read again, so that none is held
+    // through the products), then four at a time: a lane adds the products of its quarter of the row's
+    // query (as q holds the dimensions), every quarter then has the row's
+    // scores, and takes its 64 dimensions of the output through the online steps
+    // of update_online_softmax (src/attention.cpp:15-35). The row's denominator
+    // is the sum of its four lanes'. Some 30 us a tile, which the vector kernel
+    // takes 100 for on a full chip, and 8 where every row of the wave is a NaN
+    // already: nothing changes those.
+    const auto tile_in_floats = [&](uint32_t key0) {
+        float4 row_query[8][2];
+#pragma unroll
+        for (uint32_t s = 0; s < 8u; ++s) {
+            const float4 *from = reinterpret_cast<const float4 *>(query + 32u * s + 8u * quarter);
+            row_query[s][0] = from[0];
+            row_query[s][1] = from[1];
+        }
+        float4 *const key_rows = reinterpret_cast<float4 *>(key_lds);
+        float4 *const value_rows = reinterpret_cast<float4 *>(value_lds);
+        constexpr uint32_t kRow = kHeadSize / 4u;
 #pragma unroll
         for (uint32_t u = 0; u < 4u; ++u) {
-            key_in[u] = entry(keys, tile0 * kKeys + 4u * wave + u);
+            key_rows[(4u * wave + u) * kRow + lane] = entry(keys, key0 + 4u * wave + u);
+            value_rows[(4u * wave + u) * kRow + lane] = entry(values, key0 + 4u * wave + u);
+        }
+        __syncthreads();
+        const uint32_t end = min(kKeys, min(args.position + wave_token + kWaveTokens, total) - key0);
+#pragma unroll 1
+        for (uint32_t k0 = 0; k0 < end && !__all(denominator != denominator); k0 += 4u) {
+            float dot[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                const float4 *key = key_rows + (k0 + u) * kRow + 2u * quarter;
+                float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (uint32_t s = 0; s < 8u; ++s) {
+#pragma unroll
+                    for (uint32_t h = 0; h < 2u; ++h) {
+                        const float4 a = row_query[s][h], b = key[8u * s + h];
+                        sum[0] += a.x * b.x;
+                        sum[1] += a.y * b.y;
+                        sum[2] += a.z * b.z;
+                        sum[3] += a.w * b.w;
+                    }
+                }
+                dot[u] = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                dot[u] += lane_xor<16>(dot[u]);
+                dot[u] += lane_xor<32>(dot[u]);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                if (key0 + k0 + u <= seen) {
+                    const float4 *value = value_rows + (k0 + u) * kRow + 4u * quarter;
+                    const float score = dot[u] * 0.0625f;
+                    const bool up = !(score <= maximum);
+                    if (__any(up)) {
+                        const float previous = up ? expf(maximum - score) : 1.0f;
+                        maximum = up ? score : maximum;
+                        denominator *= previous;
+#pragma unroll
+                        for (uint32_t i = 0; i < 16u; ++i) {
+                            out[i] *= previous;
+                        }
+                    }
+                    const float weight = up ? 1.0f : expf(score - maximum);
+                    denominator += quarter == 0 ? weight : 0.0f;
+#pragma unroll
+                    for (uint32_t i = 0; i < 4u; ++i) {
+#pragma unroll
+                        for (uint32_t r = 0; r < 4u; ++r) {
+                            const float4 v = value[16u * i + r];
+                            out[i][r] += v.x * weight;
+                            out[i + 4u][r] += v.y * weight;
+                            out[i + 8u][r] += v.z * weight;
+                            out[i + 12u][r] += v.w * weight;
+                        }
+                    }
+                }
+            }
+        }
+    };
+
+    // runs of tiles on the matrix cores, each up to a tile that is not for them
+    uint32_t tile = tile0;
+    while (tile < tile_end) {
+        // the row's query in pieces: step s holds dimensions 32 s + 8 quarter +
+        // 0 .. 7
+        u32x4 q[8][kKeyPieces];
+        uint32_t big_query = 0;
+#pragma unroll
+        for (uint32_t s = 0; s < 8u; ++s) {
+            const float4 *from = reinterpret_cast<const float4 *>(query + 32u * s + 8u * quarter);
+            const float4 a = from[0], b = from[1];
+            big_query = largest(largest(big_query, a), b);
+            const HalfPieces c0 = split_pair_f16(a.x, a.y), c1 = split_pair_f16(a.z, a.w);
+            const HalfPieces c2 = split_pair_f16(b.x, b.y), c3 = split_pair_f16(b.z, b.w);
+            q[s][0] = u32x4{c0.hi, c1.hi, c2.hi, c3.hi};
+            q[s][1] = u32x4{c0.lo, c1.lo, c2.lo, c3.lo};
         }
 #pragma unroll
         for (uint32_t u = 0; u < 4u; ++u) {
-            value_in[u] = entry(values, tile0 * kKeys + 4u * wave + u);
+            key_in[u] = entry(keys, tile * kKeys + 4u * wave + u);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) {
+            value_in[u] = entry(values, tile * kKeys + 4u * wave + u);
         }
         __syncthreads();  // odd[] is set
         if (big_query >= kF16Overflow) {
             odd[2] = 0;
         }
-        uint32_t big = 0;
+        uint32_t first_key = 0;
 #pragma unroll
         for (uint32_t u = 0; u < 4u; ++u) {
-            big = largest(big, key_in[u]);
+            first_key = largest(first_key, key_in[u]);
             stage_key(u);
         }
-        if (big >= kF16Overflow) {
-            odd[0] = tile0;
+        if (first_key >= kF16Overflow) {
+            odd[0] = tile;
         }
-    }
-    for (uint32_t tile = tile0; tile < tile_end; ++tile) {
-        const uint32_t key0 = tile * kKeys;
-        __syncthreads();  // the tile's keys are staged; the last tile's values are free
-        // the scores, this tile's values staged between their products
-        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        // three sums a score (the small products, the large of even and of
-        // odd steps): fewer roundings at its full size
-        f32x4 small[2] = {zero, zero}, large[2][2] = {{zero, zero}, {zero, zero}};
-        uint32_t big = 0;
+        for (; tile < tile_end; ++tile) {
+            const uint32_t key0 = tile * kKeys;
+            __syncthreads();  // the tile's keys are staged; the last tile's values are free
+            // the scores, this tile's values staged between their products
+            const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+            // three sums a score (the small products, the large of even and of
+            // odd steps): fewer roundings at its full size
+            f32x4 small[2] = {zero, zero}, large[2][2] = {{zero, zero}, {zero, zero}};
+            uint32_t big = 0;
 #pragma unroll
-        for (uint32_t s = 0; s < 8u; ++s) {
+            for (uint32_t s = 0; s < 8u; ++s) {
 #pragma unroll
-            for (uint32_t m = 0; m < 2u; ++m) {
-                const unsigned char *from = key_lds + key_place(16u * m + column, 4u * s + quarter);
-                const u32x4 hi = *reinterpret_cast<const u32x4 *>(from);
-                const u32x4 lo = *reinterpret_cast<const u32x4 *>(from + kKeyPiece);
-                small[m] = mfma_f16(lo, q[s][0], small[m]);
-                small[m] = mfma_f16(hi, q[s][1], small[m]);
-                large[m][s & 1u] = mfma_f16(hi, q[s][0], large[m][s & 1u]);
-            }
-            if ((s & 1u) == 0) {
-                big = largest(big, value_in[s >> 1]);
-                stage_value(s >> 1);
-            }
-        }
-        if (big >= kBf16Overflow) {
-            odd[1] = tile;
-        }
-        const bool odd_keys = uniform(odd[0]) == tile || uniform(odd[2]) == 0;
-        __syncthreads();  // the tile's values are staged; its keys are free
-        if (odd_keys || uniform(odd[1]) == tile) {  // the same for every wave
-            exact = false;
-            break;
-        }
-        // the next tile's keys load under the softmax
-#pragma unroll
-        for (uint32_t u = 0; u < 4u; ++u) {
-            key_in[u] = entry(keys, key0 + kKeys + 4u * wave + u);
-        }
-        // score[m][r] is key key0 + 16 m + 4 quarter + r, times 1 / sqrt(256)
-        // here: in the query's pieces it would push the low ones among the
-        // subnormals
-        f32x4 score[2];
-        score[0] = ((large[0][0] + large[0][1]) + small[0]) * 0.0625f;
-        score[1] = ((large[1][0] + large[1][1]) + small[1]) * 0.0625f;
-        if (key0 + kKeys > args.position + wave_token + 1u) {  // some row of the wave ends before the tile does
-#pragma unroll
-            for (uint32_t r = 0; r < 8u; ++r) {
-                const uint32_t key = key0 + 16u * (r >> 2) + 4u * quarter + (r & 3u);
-                score[r >> 2][r & 3u] = key <= seen ? score[r >> 2][r & 3u] : -__builtin_huge_valf();
-            }
-        }
-        float top = fmaxf(fmaxf(fmaxf(score[0][0], score[0][1]), fmaxf(score[0][2], score[0][3])),
-                          fmaxf(fmaxf(score[1][0], score[1][1]), fmaxf(score[1][2], score[1][3])));
-        top = fmaxf(top, lane_xor<16>(top));
-        top = fmaxf(fmaxf(top, lane_xor<32>(top)), maximum);
-        if (__any(top > maximum)) {
-            const float factor = maximum == top ? 1.0f : expf(maximum - top);
-            denominator *= factor;
-#pragma unroll
-            for (uint32_t i = 0; i < 16u; ++i) {
-#pragma unroll
-                for (uint32_t r = 0; r < 4u; ++r) {
-                    out[i][r] *= factor;
+                for (uint32_t m = 0; m < 2u; ++m) {
+                    const unsigned char *from = key_lds + key_place(16u * m + column, 4u * s + quarter);
+                    const u32x4 hi = *reinterpret_cast<const u32x4 *>(from);
+                    const u32x4 lo = *reinterpret_cast<const u32x4 *>(from + kKeyPiece);
+                    small[m] = mfma_f16(lo, q[s][0], small[m]);
+                    small[m] = mfma_f16(hi, q[s][1], small[m]);
+                    large[m][s & 1u] = mfma_f16(hi, q[s][0], large[m][s & 1u]);
+                }
+                if ((s & 1u) == 0) {
+                    big = largest(big, value_in[s >> 1]);
+                    stage_value(s >> 1);
                 }
             }
-            maximum = top;
-        }
-        // a row with no key yet has maximum -infinity: its weights are 0
-        const float base = maximum == -__builtin_huge_valf() ? 0.0f : maximum;
-        float weight[8];
+            if (big >= kBf16Overflow) {
+                odd[1] = tile;
+            }
+            const bool odd_keys = uniform(odd[0]) == tile || uniform(odd[2]) == 0;
+            __syncthreads();  // the tile's values are staged; its keys are free
+            if (__builtin_expect(odd_keys || uniform(odd[1]) == tile, 0)) {  // the same for every wave
+                break;
+            }
+            // the next tile's keys load under the softmax
 #pragma unroll
-        for (uint32_t r = 0; r < 8u; ++r) {
-            const float s = score[r >> 2][r & 3u];
-            weight[r] = weight_of(s == base ? 0.0f : s - base);
-        }
-        denominator += ((weight[0] + weight[1]) + (weight[2] + weight[3])) +
-                       ((weight[4] + weight[5]) + (weight[6] + weight[7]));
-        // the next tile's values load under this tile's, its keys are staged
-        // between the products
+            for (uint32_t u = 0; u < 4u; ++u) {
+                key_in[u] = entry(keys, key0 + kKeys + 4u * wave + u);
+            }
+            // score[m][r] is key key0 + 16 m + 4 quarter + r, times 1 / sqrt(256)
+            // here: in the query's pieces it would push the low ones among the
+            // subnormals
+            f32x4 score[2];
+            score[0] = ((large[0][0] + large[0][1]) + small[0]) * 0.0625f;
+            score[1] = ((large[1][0] + large[1][1]) + small[1]) * 0.0625f;
+            if (key0 + kKeys > args.position + wave_token + 1u) {  // some row of the wave ends before the tile does
 #pragma unroll
-        for (uint32_t u = 0; u < 4u; ++u) {
-            value_in[u] = entry(values, key0 + kKeys + 4u * wave + u);
-        }
-        u32x4 p[kPieces];
-        {
-            const Pieces c0 = split_pair(weight[0], weight[1]), c1 = split_pair(weight[2], weight[3]);
-            const Pieces c2 = split_pair(weight[4], weight[5]), c3 = split_pair(weight[6], weight[7]);
+                for (uint32_t r = 0; r < 8u; ++r) {
+                    const uint32_t key = key0 + 16u * (r >> 2) + 4u * quarter + (r & 3u);
+                    score[r >> 2][r & 3u] = key <= seen ? score[r >> 2][r & 3u] : -__builtin_huge_valf();
+                }
+            }
+            float top = fmaxf(fmaxf(fmaxf(score[0][0], score[0][1]), fmaxf(score[0][2], score[0][3])),
+                              fmaxf(fmaxf(score[1][0], score[1][1]), fmaxf(score[1][2], score[1][3])));
+            top = fmaxf(top, lane_xor<16>(top));
+            top = fmaxf(fmaxf(top, lane_xor<32>(top)), maximum);
+            if (__any(top > maximum)) {
+                const float factor = maximum == top ? 1.0f : expf(maximum - top);
+                denominator *= factor;
 #pragma unroll
-            for (uint32_t i = 0; i < kPieces; ++i) {
-                p[i] = u32x4{c0.p[i], c1.p[i], c2.p[i], c3.p[i]};
+                for (uint32_t i = 0; i < 16u; ++i) {
+#pragma unroll
+                    for (uint32_t r = 0; r < 4u; ++r) {
+                        out[i][r] *= factor;
+                    }
+                }
+                maximum = top;
+            }
+            // a row with no key yet has maximum -infinity: its weights are 0
+            const float base = maximum == -__builtin_huge_valf() ? 0.0f : maximum;
+            float weight[8];
+#pragma unroll
+            for (uint32_t r = 0; r < 8u; ++r) {
+                const float s = score[r >> 2][r & 3u];
+                weight[r] = weight_of(s == base ? 0.0f : s - base);
+            }
+            denominator += ((weight[0] + weight[1]) + (weight[2] + weight[3])) +
+                           ((weight[4] + weight[5]) + (weight[6] + weight[7]));
+            // the next tile's values load under this tile's, its keys are staged
+            // between the products
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                value_in[u] = entry(values, key0 + kKeys + 4u * wave + u);
+            }
+            u32x4 p[kPieces];
+            {
+                const Pieces c0 = split_pair(weight[0], weight[1]), c1 = split_pair(weight[2], weight[3]);
+                const Pieces c2 = split_pair(weight[4], weight[5]), c3 = split_pair(weight[6], weight[7]);
+#pragma unroll
+                for (uint32_t i = 0; i < kPieces; ++i) {
+                    p[i] = u32x4{c0.p[i], c1.p[i], c2.p[i], c3.p[i]};
+                }
+            }
+            uint32_t next_key = 0;
+#pragma unroll
+            for (uint32_t i = 0; i < 16u; ++i) {
+                u32x4 v[kPieces];
+#pragma unroll
+                for (uint32_t k = 0; k < kPieces; ++k) {
+                    v[k] = *reinterpret_cast<const u32x4 *>(value_lds + k * kValuePiece +
+                                                            value_place(16u * i + column, quarter));
+                }
+                out[i] = product(v, p, out[i]);
+                if ((i & 3u) == 0) {
+                    next_key = largest(next_key, key_in[i >> 2]);
+                    stage_key(i >> 2);
+                }
+            }
+            if (next_key >= kF16Overflow) {
+                odd[0] = tile + 1u;
             }
         }
-        big = 0;
-#pragma unroll
-        for (uint32_t i = 0; i < 16u; ++i) {
-            u32x4 v[kPieces];
-#pragma unroll
-            for (uint32_t k = 0; k < kPieces; ++k) {
-                v[k] = *reinterpret_cast<const u32x4 *>(value_lds + k * kValuePiece +
-                                                        value_place(16u * i + column, quarter));
-            }
-            out[i] = product(v, p, out[i]);
-            if ((i & 3u) == 0) {
-                big = largest(big, key_in[i >> 2]);
-                stage_key(i >> 2);
-            }
+        if (__builtin_expect(tile < tile_end, 0)) {
+            tile_in_floats(tile * kKeys);
+            ++tile;
         }
-        if (big >= kF16Overflow) {
-            odd[0] = tile + 1u;
-        }
-    }
-
-    if (!exact) {
-        rows_in_floats(args, kv, split, wave_token, tile0 * kKeys, tile_end * kKeys);
-        return;
     }
     denominator += lane_xor<16>(denominator);
     denominator += lane_xor<32>(denominator);

@@ -81,20 +81,32 @@ def test_attention_chunk_edges(gpu, oracle, tluts, position, count):
         assert max_rel_error(out[b].cpu().numpy(), want) <= 1e-4, b
 
 
-@pytest.mark.parametrize("case", ["token", "key", "value", "large"])
+@pytest.mark.parametrize("case", ["token", "key", "value", "large", "query", "unseen"])
 def test_attention_chunk_odd_values(gpu, tluts, case):
     """Values the matrix cores' pieces cannot stand for: a NaN token (its row
     and those after it are NaN, those before it are not), an infinity in the
-    history's keys or values, and finite values beyond f16 and bf16 give what
-    the vector kernel (chunks of 8 tokens) gives."""
+    history's keys or values, finite values beyond f16 and bf16, a query of 2^62,
+    and keys of 2^70 in the first, a middle, the last whole and the chunk's own
+    tile where the query is 0, so that tiles in floats and on the matrix cores
+    take turns at one softmax, give what the vector kernel (chunks of 8 tokens)
+    gives."""
     rng = syn.rng_for(67, len(case))
     layer = syn.full_attention(rng, HIDDEN, tluts[1])
+    if case == "query":
+        layer.query_norm[100] = 0x5E80  # 2^62 in bf16
+    elif case == "unseen":
+        layer.query_norm[100] = 0xBF80  # -1: times 0
     d = hip.upload_full_attention(gpu, layer, gpu.ne_codebook(tluts[1]))
     position, count = 600, 40
     keys = rng.normal(0.0, 1.0, (position + count, 2, 256)).astype(np.float32)
     values = rng.normal(0.0, 1.0, (position + count, 2, 256)).astype(np.float32)
     x = syn.rms_normalized(syn.hidden_states(rng, count, HIDDEN))
-    if case == "token":
+    if case == "unseen":
+        keys[[5, 300, 575, 599], :, 100] = 2.0 ** 70
+        keys[64:96, :, 100] = -2.0 ** 70
+    elif case == "query":
+        pass
+    elif case == "token":
         x[21, 5] = np.nan
     elif case == "key":
         keys[70, 0, 9] = np.inf

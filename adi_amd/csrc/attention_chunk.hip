@@ -14,27 +14,35 @@
 //
 // Precision: operands are split so that the matrix cores' 16-bit products add
 // up to a float product's accuracy, in float accumulators. Queries and keys
-// take two f16 pieces (round to nearest: 22 significant bits and a sign, an
-// absolute 2^-25 for the smallest) and the three products without lo lo,
-// below 2^-24 of a product; a score's error is absolute in the softmax, so
-// small keys need no more. Probabilities and values take three bf16 pieces
-// that sum to them exactly, at any scale, and the six products down to 2^-16;
-// what is left out is below 2^-25 of a product. Against 64 bits the layer's
-// output is as far off as with the vector kernel: 1.231e-6 and 1.233e-6 for
-// 512 tokens at position 3584, 7.35e-7 and 7.47e-7 for 64 at 1000, 8.24e-7 and
-// 8.19e-7 for 128 at 0 (relative, the projections' part included).
+// take two f16 pieces (round to nearest: 22 significant bits and a sign) and
+// the three products without lo lo, which is below 2^-22 of a product. f16's
+// range is small, so they are scaled first, by an exact power of two for a
+// query row and for each four keys (a wave's), to a largest value of 2^14 to
+// 2^15, and the scores scaled back: the low pieces' absolute floor of 2^-25 is
+// then 2^-39 of the largest. (The scales cost 6 us of 177; unscaled, queries of
+// 2^13 over keys of 2^-13 came out 1e-4 off.) Probabilities and values take
+// three bf16 pieces that sum to them exactly, at any scale, and the six products
+// down to 2^-16; what is left out is below 2^-25 of a product. Against 64 bits
+// the layer's output is as far off as with the vector kernel: 1.231e-6 and
+// 1.233e-6 for 512 tokens at position 3584, 7.35e-7 and 7.47e-7 for 64 at 1000,
+// 8.24e-7 and 8.19e-7 for 128 at 0 (relative, the projections' part included);
+// with queries and keys of 2^-30 to 2^30, 64 at 1000 and 256 hidden values, 4.8
+// to 6.2e-7 and 4.8 to 6.1e-7.
 //
 // What bounds it: the matrix cores are busy 45% of the time, the LDS (every
 // wave reads every staged entry) 30%, vector issue (the splits, the softmax)
-// 45%, in phases between barriers. 512 tokens at position 3584: 178 us, the
+// 45%, in phases between barriers. 512 tokens at position 3584: 177 us, the
 // vector kernel 3048 (each query head of each token read the history again).
 // Four waves of 32 rows with v_mfma_f32_32x32x16, one a SIMD: 200 us.
 //
-// A tile with a value the pieces cannot stand for (an infinity, a NaN, a query
-// or key that rounds to an f16 infinity) runs in plain floats, entry by entry,
-// on the same running state: a row skips the entries behind its position, which
-// a matrix product multiplies by zero.
+// A tile with a value the pieces cannot stand for (an infinity, a NaN, 2^60 and
+// more in a key or query, whose scores could overflow) runs in plain floats,
+// entry by entry, on the same running state: a row skips the entries behind its
+// position, which a matrix product multiplies by zero. A query row with a NaN
+// is NaN either way and stays on the matrix cores.
 #include "attention.hpp"
+
+#include <type_traits>
 
 namespace adi_hip {
 namespace {
@@ -63,10 +71,12 @@ __device__ __forceinline__ uint32_t value_place(uint32_t row, uint32_t piece) {
     return row * kValuePitch + ((piece ^ ((0x78u >> ((row >> 1) & 6u)) & 3u)) << 4);
 }
 constexpr uint32_t kStaged = kKeyPieces * kKeyPiece + kPieces * kValuePiece;
-constexpr uint32_t kChunkLds = kStaged + 16;
-// the smallest float bits that round to an infinity in f16 and bf16
-constexpr uint32_t kF16Overflow = 0x477FF000u;
+constexpr uint32_t kChunkLds = kStaged + 16 + kThreads / 64u * 4u;
+// the smallest float bits that round to an infinity in bf16, those of 2^60, and
+// of infinity
 constexpr uint32_t kBf16Overflow = 0x7F7F8000u;
+constexpr uint32_t kScoreLimit = (127u + 60u) << 23;
+constexpr uint32_t kInfinity = 0x7F800000u;
 constexpr uint32_t kNoTile = 0xFFFFFFFFu;
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -145,12 +155,36 @@ __device__ __forceinline__ float weight_of(float d) {
     return fmaf(y * tail, kLn2, y);
 }
 
+// The power of two that brings values of a largest magnitude of these float
+// bits (below infinity) to 2^14 .. 2^15, and its inverse; 2^126 at most.
+__device__ __forceinline__ uint32_t scale_exponent(uint32_t largest) { return min(268u - (largest >> 23), 253u); }
+__device__ __forceinline__ float scale_of(uint32_t exponent) { return __uint_as_float(exponent << 23); }
+__device__ __forceinline__ float unscale_of(uint32_t exponent) { return __uint_as_float((254u - exponent) << 23); }
+
+// The largest of the wave's values, a scalar.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+    const auto rotated = [](uint32_t x, auto control) {
+        return static_cast<uint32_t>(
+            __builtin_amdgcn_mov_dpp(static_cast<int>(x), decltype(control)::value, 0xF, 0xF, true));
+    };
+    v = max(v, rotated(v, std::integral_constant<int, 0x128>{}));  // row_ror:8
+    v = max(v, rotated(v, std::integral_constant<int, 0x124>{}));  // row_ror:4
+    v = max(v, rotated(v, std::integral_constant<int, 0x122>{}));  // row_ror:2
+    v = max(v, rotated(v, std::integral_constant<int, 0x121>{}));  // row_ror:1
+    const auto row = [&](int lane) {
+        return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), lane));
+    };
+    return max(max(row(0), row(16)), max(row(32), row(48)));
+}
+
 __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args) {
     extern __shared__ __align__(16) unsigned char lds[];
     unsigned char *const key_lds = lds;
     unsigned char *const value_lds = lds + kKeyPieces * kKeyPiece;
     // the last tile with an unsplittable key, and value, and whether a query is
     volatile uint32_t *const odd = reinterpret_cast<volatile uint32_t *>(lds + kStaged);
+    // what takes the scores of keys 4 w .. 4 w + 3 back from their scale
+    volatile float *const key_unscale = reinterpret_cast<volatile float *>(lds + kStaged + 16);
     // blocks of one (KV head, split) read the same entries: with 8 or more
     // such pairs each stays on one XCD (block b runs on XCD b % 8)
     const uint32_t pairs = kKvHeads * args.splits;
@@ -192,9 +226,23 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
         return reinterpret_cast<const float4 *>(cache + static_cast<size_t>(min(key, total - 1u)) * kKvHeads *
                                                             kHeadSize)[lane];
     };
+    // the largest of the wave's four keys of a tile, and what takes its scale
+    // back into LDS
+    const auto largest_key = [&] {
+        uint32_t big = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) {
+            big = largest(big, key_in[u]);
+        }
+        big = wave_max(big);
+        key_unscale[wave] = unscale_of(scale_exponent(min(big, kScoreLimit)));
+        return big;
+    };
+    const auto key_scale = [](uint32_t big) { return scale_of(scale_exponent(min(big, kScoreLimit))); };
     // key row 4 wave + u into LDS
-    const auto stage_key = [&](uint32_t u) {
-        const HalfPieces a = split_pair_f16(key_in[u].x, key_in[u].y), b = split_pair_f16(key_in[u].z, key_in[u].w);
+    const auto stage_key = [&](uint32_t u, float scale) {
+        const HalfPieces a = split_pair_f16(key_in[u].x * scale, key_in[u].y * scale);
+        const HalfPieces b = split_pair_f16(key_in[u].z * scale, key_in[u].w * scale);
         unsigned char *to = key_lds + key_place(4u * wave + u, lane >> 1) + 8u * (lane & 1u);
         *reinterpret_cast<uint2 *>(to) = make_uint2(a.hi, b.hi);
         *reinterpret_cast<uint2 *>(to + kKeyPiece) = make_uint2(a.lo, b.lo);
@@ -313,13 +361,27 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
         // 0 .. 7
         u32x4 q[8][kKeyPieces];
         uint32_t big_query = 0;
+        float4 query_in[8][2];
 #pragma unroll
         for (uint32_t s = 0; s < 8u; ++s) {
             const float4 *from = reinterpret_cast<const float4 *>(query + 32u * s + 8u * quarter);
-            const float4 a = from[0], b = from[1];
-            big_query = largest(largest(big_query, a), b);
-            const HalfPieces c0 = split_pair_f16(a.x, a.y), c1 = split_pair_f16(a.z, a.w);
-            const HalfPieces c2 = split_pair_f16(b.x, b.y), c3 = split_pair_f16(b.z, b.w);
+            query_in[s][0] = from[0];
+            query_in[s][1] = from[1];
+            big_query = largest(largest(big_query, query_in[s][0]), query_in[s][1]);
+        }
+        big_query = max(big_query, lane_xor_bits<16>(big_query));
+        big_query = max(big_query, lane_xor_bits<32>(big_query));
+        const uint32_t query_exponent = scale_exponent(min(big_query, kScoreLimit));
+        const float query_scale = scale_of(query_exponent);
+        // with 1 / sqrt(256)
+        const float query_unscale = unscale_of(query_exponent) * 0.0625f;
+#pragma unroll
+        for (uint32_t s = 0; s < 8u; ++s) {
+            const float4 a = query_in[s][0], b = query_in[s][1];
+            const HalfPieces c0 = split_pair_f16(a.x * query_scale, a.y * query_scale);
+            const HalfPieces c1 = split_pair_f16(a.z * query_scale, a.w * query_scale);
+            const HalfPieces c2 = split_pair_f16(b.x * query_scale, b.y * query_scale);
+            const HalfPieces c3 = split_pair_f16(b.z * query_scale, b.w * query_scale);
             q[s][0] = u32x4{c0.hi, c1.hi, c2.hi, c3.hi};
             q[s][1] = u32x4{c0.lo, c1.lo, c2.lo, c3.lo};
         }
@@ -332,16 +394,15 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
             value_in[u] = entry(values, tile * kKeys + 4u * wave + u);
         }
         __syncthreads();  // odd[] is set
-        if (big_query >= kF16Overflow) {
+        if (big_query >= kScoreLimit && big_query <= kInfinity) {
             odd[2] = 0;
         }
-        uint32_t first_key = 0;
+        const uint32_t first_key = largest_key();
 #pragma unroll
         for (uint32_t u = 0; u < 4u; ++u) {
-            first_key = largest(first_key, key_in[u]);
-            stage_key(u);
+            stage_key(u, key_scale(first_key));
         }
-        if (first_key >= kF16Overflow) {
+        if (first_key >= kScoreLimit) {
             odd[0] = tile;
         }
         for (; tile < tile_end; ++tile) {
@@ -373,6 +434,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
                 odd[1] = tile;
             }
             const bool odd_keys = uniform(odd[0]) == tile || uniform(odd[2]) == 0;
+            const float unscale[2] = {key_unscale[quarter], key_unscale[4u + quarter]};
             __syncthreads();  // the tile's values are staged; its keys are free
             if (__builtin_expect(odd_keys || uniform(odd[1]) == tile, 0)) {  // the same for every wave
                 break;
@@ -382,12 +444,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
             for (uint32_t u = 0; u < 4u; ++u) {
                 key_in[u] = entry(keys, key0 + kKeys + 4u * wave + u);
             }
-            // score[m][r] is key key0 + 16 m + 4 quarter + r, times 1 / sqrt(256)
-            // here: in the query's pieces it would push the low ones among the
-            // subnormals
+            // score[m][r] is key key0 + 16 m + 4 quarter + r
             f32x4 score[2];
-            score[0] = ((large[0][0] + large[0][1]) + small[0]) * 0.0625f;
-            score[1] = ((large[1][0] + large[1][1]) + small[1]) * 0.0625f;
+            score[0] = ((large[0][0] + large[0][1]) + small[0]) * (query_unscale * unscale[0]);
+            score[1] = ((large[1][0] + large[1][1]) + small[1]) * (query_unscale * unscale[1]);
             if (key0 + kKeys > args.position + wave_token + 1u) {  // some row of the wave ends before the tile does
 #pragma unroll
                 for (uint32_t r = 0; r < 8u; ++r) {
@@ -446,12 +506,14 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
                                                             value_place(16u * i + column, quarter));
                 }
                 out[i] = product(v, p, out[i]);
+                if (i == 0) {
+                    next_key = largest_key();
+                }
                 if ((i & 3u) == 0) {
-                    next_key = largest(next_key, key_in[i >> 2]);
-                    stage_key(i >> 2);
+                    stage_key(i >> 2, key_scale(next_key));
                 }
             }
-            if (next_key >= kF16Overflow) {
+            if (next_key >= kScoreLimit) {
                 odd[0] = tile + 1u;
             }
         }

@@ -61,10 +61,9 @@ def test_attention_chunk_edges(gpu, oracle, tluts, position, count):
     """The matrix-core attention of a chunk at the edges of its 16-token
     blocks and 32-key tiles, with one and several splits, against the oracle's
     one-token form for the first, last and middle tokens (the caches as the
-    chunk left them). Scores and weights carry a float's relative error
-    (2^-22 at most per product), so outputs agree to the float noise of 32-bit
-    sums of up to 4020 terms: 1e-4 of the largest covers 4020 * 2^-24 = 2.4e-4
-    at a quarter of its worst case, as in the one-token tests."""
+    chunk left them). Both sides sum in floats; the largest difference seen is
+    2.9e-6 of the largest output (20 tokens at 4000), and 1e-5 is about four
+    times that. test_attention_chunk_precision holds the pieces to 64 bits."""
     rng = syn.rng_for(66, position + count)
     layer = syn.full_attention(rng, HIDDEN, tluts[1])
     d = hip.upload_full_attention(gpu, layer, gpu.ne_codebook(tluts[1]))
@@ -78,7 +77,7 @@ def test_attention_chunk_edges(gpu, oracle, tluts, position, count):
     keys, values = dk.cpu().numpy(), dv.cpu().numpy()
     for b in sorted({0, 1, 15, count // 2, count - 1}):
         want = po.full_attention_forward(oracle, held, position + b, x[b], keys.copy(), values.copy())
-        assert max_rel_error(out[b].cpu().numpy(), want) <= 1e-4, b
+        assert max_rel_error(out[b].cpu().numpy(), want) <= 1e-5, b
 
 
 @pytest.mark.parametrize("case", ["token", "key", "value", "large", "query", "unseen"])
@@ -131,6 +130,117 @@ def test_attention_chunk_odd_values(gpu, tluts, case):
     for a, b in zip(got, want):
         if np.isfinite(b).all():
             assert max_rel_error(a, b) <= 1e-4
+
+
+def hadamard64(v):
+    n, lead, h = v.shape[-1], v.shape[:-1], 1
+    while h < n:
+        v = v.reshape(*lead, n // (2 * h), 2, h)
+        v = np.stack((v[..., 0, :] + v[..., 1, :], v[..., 0, :] - v[..., 1, :]), -2)
+        h *= 2
+    return v.reshape(*lead, n) / np.sqrt(n)
+
+
+def ne64(m, x):
+    """An NE projection in 64 bits: 16-bit windows of each tile's 64 words, one
+    every 8 bits, through the state table."""
+    w = np.asarray(m.trellis).astype(np.int64).reshape(-1, 64) & 0xFFFF
+    at = np.arange(128) * 8
+    pair = (w[:, at // 16] << 16) | w[:, (at // 16 + 1) % 64]
+    state = (pair >> (16 - at % 16)) & 0xFFFF
+    product = state * (state + 1)
+    v = np.asarray(m.tlut, np.float64).astype(np.float16).astype(np.float64).reshape(512, 2)[(product >> 6) & 0x1FF]
+    v[..., 0] *= 1.0 - 2.0 * ((product >> 15) & 1)
+    dense = v.reshape(m.rows // 16, m.columns // 16, 16, 16).transpose(0, 2, 1, 3).reshape(m.rows, m.columns)
+    return hadamard64(hadamard64(x * np.asarray(m.su, np.float64)) @ dense.T * m.weight_scale) * np.asarray(m.sv, np.float64)
+
+
+def full_attention64(layer, position, x, keys, values, planted=None):
+    """A chunk's attention in 64 bits over the history keys[:position],
+    values[:position]; `planted` changes (weights, values) before their product."""
+    n = len(x)
+    positions = np.arange(position, position + n)
+    bf16 = lambda bits: (bits.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    angle = (positions.astype(np.float32)[:, None]
+             / np.power(1e7, np.arange(32) / 32.0).astype(np.float32)).astype(np.float64)[:, None]
+
+    def norm_rope(v, weight):
+        v = v / np.sqrt((v * v).mean(-1, keepdims=True) + 1e-6) * (1.0 + bf16(weight))
+        c, s = np.cos(angle), np.sin(angle)
+        return np.concatenate((v[..., :32] * c - v[..., 32:64] * s, v[..., 32:64] * c + v[..., :32] * s, v[..., 64:]), -1)
+
+    qg = ne64(layer.query, x).reshape(n, 16, 2, 256)
+    q, gate = norm_rope(qg[:, :, 0], layer.query_norm), qg[:, :, 1]
+    k = np.concatenate((keys[:position], norm_rope(ne64(layer.key, x).reshape(n, 2, 256), layer.key_norm)))
+    v = np.concatenate((values[:position], ne64(layer.value, x).reshape(n, 2, 256)))
+    attended = np.empty((n, 16, 256))
+    for h in range(16):
+        s = q[:, h] @ k[:, h // 8].T / 16.0
+        s[np.arange(position + n)[None] > positions[:, None]] = -np.inf
+        w = np.exp(s - s.max(1, keepdims=True))
+        held = v[:, h // 8]
+        if planted is not None:
+            w, held = planted(w, held)
+        attended[:, h] = w @ held / w.sum(1, keepdims=True)
+    return ne64(layer.output, (attended / (1.0 + np.exp(-gate))).reshape(n, -1))
+
+
+# The query and key scales of the chunk attention's precision test: the query
+# norm's weight (a scale of 1 + w), the scale of the history's keys, and a scale
+# of dimension 100's keys with the query's norm weight there.
+PRECISION = {
+    "flat": (-1 + 2.0 ** -4, 1.0, None), "unit": (0.0, 1.0, None), "low keys": (255.0, 2.0 ** -8, None),
+    "lower keys": (2.0 ** 13, 2.0 ** -13, None), "lowest keys": (2.0 ** 30, 2.0 ** -30, None),
+    "high keys": (-1 + 2.0 ** -8, 2.0 ** 8, None),
+    "one dimension": (255.0, 2.0 ** -8, (2.0 ** 8, -1 + 2.0 ** -8))}
+
+
+def precision_case(tlut, name):
+    """Layer, position, tokens and history of a case. The fresh keys are 0 (their
+    norm weight is -1), so that scores come from the history's scale alone."""
+    weight, scale, dimension = PRECISION[name]
+    rng = syn.rng_for(68, sorted(PRECISION).index(name))
+    layer = syn.full_attention(rng, HIDDEN, tlut)
+    bf16 = lambda v: np.array([v], np.float32).view(np.uint32)[0] >> 16
+    layer.query_norm[:] = bf16(weight)
+    layer.key_norm[:] = bf16(-1.0)
+    position, count = 1000, 64
+    keys = rng.normal(0.0, scale, (position + count, 2, 256)).astype(np.float32)
+    values = rng.normal(0.0, 1.0, (position + count, 2, 256)).astype(np.float32)
+    if dimension is not None:
+        keys[:, :, 100] *= dimension[0] / scale
+        layer.query_norm[100] = bf16(dimension[1])
+    return layer, position, syn.rms_normalized(syn.hidden_states(rng, count, HIDDEN)), keys, values
+
+
+def two_bf16_pieces(v):
+    """v rounded to bf16 plus the rest rounded to bf16."""
+    v, out = np.asarray(v, np.float32), 0.0
+    for _ in range(2):
+        bits = (v - np.float32(out)).view(np.uint32)
+        out = out + ((bits + 0x7FFF + ((bits >> 16) & 1)) & 0xFFFF0000).astype(np.uint32).view(np.float32)
+    return out.astype(np.float64)
+
+
+@pytest.mark.parametrize("name", list(PRECISION))
+def test_attention_chunk_precision(gpu, tluts, name):
+    """The layer's error against 64 bits at query and key scales from 2^-30 to
+    2^30, and with one dimension's keys 2^16 times the others'. The projections'
+    part is about 5e-7 (relative, 2-norm), which the vector kernel shows too; the
+    bound is twice the 6.2e-7 seen. Weights or values in two pieces instead of
+    three, planted in the 64-bit form, are past it by half, and pieces of
+    unscaled keys were 3e-6 to 1e-4 off."""
+    bound = 1.25e-6
+    layer, position, x, keys, values = precision_case(tluts[1], name)
+    want = full_attention64(layer, position, x, keys, values)
+    error = lambda got: np.linalg.norm(got - want) / np.linalg.norm(want)
+    for planted in (lambda w, v: (two_bf16_pieces(w), v), lambda w, v: (w, two_bf16_pieces(v))):
+        assert error(full_attention64(layer, position, x, keys, values, planted)) > 1.5 * bound
+    d = hip.upload_full_attention(gpu, layer, gpu.ne_codebook(tluts[1]))
+    dk, dv = dev(keys), dev(values)
+    out = torch.empty((len(x), HIDDEN), dtype=torch.float32, device="cuda")
+    hip.full_attention_prefill(gpu, d, position, len(x), dev(x), out, dk, dv, len(keys))
+    assert error(out.cpu().numpy()) <= bound
 
 
 def test_linear_attention_prefill(gpu, oracle, tluts):

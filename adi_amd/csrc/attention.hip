@@ -359,6 +359,7 @@ struct RowsLds {
     __align__(16) float query[kHeadsPerKv][kQueryPad];
     __align__(16) float acc[4][kHeadsPerKv][kMergePad];
     float maximum[4][kHeadsPerKv], denominator[4][kHeadsPerKv];
+    float factor[kHeadsPerKv][4], top[kHeadsPerKv];
     uint32_t odd;
 };
 
@@ -366,6 +367,9 @@ struct RowsLds {
 // query heads (lds.query) by a block of four waves, wave w taking every fourth
 // tile of kTile entries, and the split's part of each head to partial (written
 // through to memory with COHERENT: a later block of the same launch reads it).
+// With `attended` (a row of one part) each head's output, times its sigmoid
+// gate at query_gate, goes there instead, unless a score is not a number.
+// Returns whether it went to partial.
 //
 // A tile is two chains of v_mfma_f32_16x16x4_f32 in which a lane's registers
 // are loaded as the matrix core reads them, straight from the cache: the
@@ -381,11 +385,15 @@ struct RowsLds {
 // chain of norm, tile and merge where they are few. One head's wave at a time
 // over float registers (a wave sum and an exponential a head and entry, each
 // entry read eight times) took 201 us for 32 rows at up to 2,000 entries, this
-// 62 (131 MB: 2.1 TB/s), and one row at 2,000 27.1 and 21.3.
+// 62 (131 MB: 2.1 TB/s); one row at 40, 200, 400 and 2,000 entries 10.8, 11.5,
+// 13.6, 27.6 and 10.1, 14.4, 14.4, 19.7 (a row of one part without the round
+// trip through memory, 12.8 with it; every thread taking the waves' factors of
+// every head itself cost 1.7 more).
 template <bool COHERENT>
-__device__ __forceinline__ void attention_rows_span(RowsLds &lds, const float *keys, const float *values,
+__device__ __forceinline__ bool attention_rows_span(RowsLds &lds, const float *keys, const float *values,
                                                     uint32_t tokens, uint32_t chunk, float *partial, uint32_t kv,
-                                                    uint32_t split, uint32_t splits) {
+                                                    uint32_t split, uint32_t splits, const float *query_gate = nullptr,
+                                                    float *attended = nullptr) {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t c = lane & 15u, g = lane >> 4;
     const uint32_t begin = split * chunk;
@@ -525,22 +533,45 @@ __device__ __forceinline__ void attention_rows_span(RowsLds &lds, const float *k
                                              kv * kHeadsPerKv + h, split, splits);
             __syncthreads();
         }
-        return;
+        return true;
+    }
+    // each wave's factor of each head by one thread, not by all
+    if (threadIdx.x < 4u * kHeadsPerKv) {
+        const uint32_t h = threadIdx.x % kHeadsPerKv, w = threadIdx.x / kHeadsPerKv;
+        const float m = fmaxf(fmaxf(lds.maximum[0][h], lds.maximum[1][h]), fmaxf(lds.maximum[2][h], lds.maximum[3][h]));
+        // 0 for a wave without tokens, and where no wave has any
+        lds.factor[h][w] = m != -__builtin_huge_valf() ? expf(lds.maximum[w][h] - m) : 0.0f;
+        lds.top[h] = m;
+    }
+    __syncthreads();
+    const auto merged = [&](uint32_t h, float &a, float &d) {
+        a = 0.0f;
+        d = 0.0f;
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) {
+            a += lds.acc[w][h][threadIdx.x] * lds.factor[h][w];
+            d += lds.denominator[w][h] * lds.factor[h][w];
+        }
+    };
+    if (attended != nullptr) {  // uniform; the combine of one part
+        float gate[kHeadsPerKv];
+#pragma unroll
+        for (uint32_t h = 0; h < kHeadsPerKv; ++h) {
+            gate[h] = query_gate[h * kQueryStride + kHeadSize + threadIdx.x];
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < kHeadsPerKv; ++h) {
+            float a, d;
+            merged(h, a, d);
+            attended[h * kHeadSize + threadIdx.x] = a * (1.0f / d) * sigmoid_of(gate[h]);
+        }
+        return false;
     }
 #pragma unroll
     for (uint32_t h = 0; h < kHeadsPerKv; ++h) {
-        float m = lds.maximum[0][h];
-        for (uint32_t w = 1; w < 4; ++w) {
-            m = fmaxf(m, lds.maximum[w][h]);
-        }
-        float a = 0.0f, d = 0.0f;
-        if (m != -__builtin_huge_valf()) {  // else no token in this split
-            for (uint32_t w = 0; w < 4; ++w) {
-                const float f = expf(lds.maximum[w][h] - m);  // 0 for a wave without tokens
-                a += lds.acc[w][h][threadIdx.x] * f;
-                d += lds.denominator[w][h] * f;
-            }
-        }
+        const float m = lds.top[h];
+        float a, d;
+        merged(h, a, d);
         float *out = partial + (static_cast<size_t>(kv * kHeadsPerKv + h) * splits + split) * kPartialStride;
         if constexpr (COHERENT) {
             coherent_store(out + threadIdx.x, a);
@@ -556,6 +587,7 @@ __device__ __forceinline__ void attention_rows_span(RowsLds &lds, const float *k
             }
         }
     }
+    return true;
 }
 
 // Row r of a decode step over sequences sees its own cache's entries
@@ -713,16 +745,21 @@ __global__ __launch_bounds__(256, 2) void k_attention_rows_one(const float *quer
         norm_rope_wave(query_gate + (head + h) * kQueryStride, lds.query[h], query_norm, rope);
     }
     if (split == parts.splits - 1u) {  // uniform over the block
+        // (ahead of the queries, which its way to memory then overlaps)
         const size_t src = (static_cast<size_t>(r) * kKvHeads + kv) * kHeadSize;
         const size_t entry = (static_cast<size_t>(position) * kKvHeads + kv) * kHeadSize;
+        rows.values[r][entry + t] = value[src + t];
         if (wave == 0u) {
             norm_rope_wave(key + src, rows.keys[r] + entry, key_norm, rope);
         }
-        rows.values[r][entry + t] = value[src + t];
     }
     __syncthreads();  // the block reads back its own entry
     float *p = partial + static_cast<size_t>(r) * kQueryHeads * grid_splits * kPartialStride;
-    attention_rows_span<true>(lds, rows.keys[r], rows.values[r], tokens, parts.chunk, p, kv, split, grid_splits);
+    const bool one = parts.splits == 1u;
+    if (!attention_rows_span<true>(lds, rows.keys[r], rows.values[r], tokens, parts.chunk, p, kv, split, grid_splits,
+                                   query_gate + head * kQueryStride, one ? attended + head * kHeadSize : nullptr)) {
+        return;
+    }
     wait_stores();
     __syncthreads();
     uint32_t *ticket = tickets + static_cast<size_t>(r) * kQueryHeads + kv;

@@ -68,8 +68,8 @@ struct FullRows {
 // depend on the launch's grid (any grid with at least this many parts gives the
 // same bits) or on the other rows. A short history takes one tile a wave, the
 // shortest chain; past kShortHistory entries two tiles a wave, which halves the
-// parts to write and merge (one row at 600 entries: 17.6 us with one tile, 19.9
-// with two; at 4096 28.0 and 24.7; 16 rows at up to 4096 69 and 62).
+// parts to write and merge (one row at 600 entries: 15.9 us with one tile, 18.0
+// with two; at 4096 26.5 and 23.1; 16 rows at up to 4096 64 and 60).
 constexpr uint32_t kTile = 16;
 constexpr uint32_t kShortHistory = 1024;
 constexpr uint32_t kRowPartials = 1024, kLeastPartials = 64;  // parts of all rows
@@ -368,7 +368,7 @@ struct RowsLds {
 // tile of kTile entries, and the split's part of each head to partial (written
 // through to memory with COHERENT: a later block of the same launch reads it).
 // With `attended` (a row of one part) each head's output, times its sigmoid
-// gate at query_gate, goes there instead, unless a score is not a number.
+// gate at query_gate, goes there instead, unless a score is infinite.
 // Returns whether it went to partial.
 //
 // A tile is two chains of v_mfma_f32_16x16x4_f32 in which a lane's registers
@@ -456,7 +456,7 @@ __device__ __forceinline__ bool attention_rows_span(RowsLds &lds, const float *k
         f32x4 p = ((s[0] + s[1]) + (s[2] + s[3])) * (1.0f / 16.0f);  // 1 / sqrt(256)
 #pragma unroll
         for (uint32_t r = 0; r < 4; ++r) {
-            odd |= !(fabsf(p[r]) < __builtin_huge_valf());
+            odd |= fabsf(p[r]) == __builtin_huge_valf();
         }
         if (ragged) {
 #pragma unroll
@@ -527,7 +527,10 @@ __device__ __forceinline__ bool attention_rows_span(RowsLds &lds, const float *k
         }
     }
     __syncthreads();
-    if (lds.odd != 0u) {  // uniform: a score that is not a number, head by head
+    // uniform: an infinite score, whose row goes entry by entry, head by head.
+    // (One that is a NaN stays: it leaves NaNs in its head's denominator and
+    // accumulator whatever the factors are, as it does entry by entry.)
+    if (lds.odd != 0u) {
         for (uint32_t h = 0; h < kHeadsPerKv; ++h) {
             attention_partial_span<COHERENT>(lds.query[h], keys, values, tokens, chunk, partial,
                                              kv * kHeadsPerKv + h, split, splits);

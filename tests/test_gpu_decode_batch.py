@@ -245,6 +245,47 @@ def test_decode_batch_history_edges(gpu, parts, limit):
             assert np.isfinite(want).all() and max_rel_error(one[b], want) <= 1e-3, (b, positions[b])
 
 
+@pytest.mark.parametrize("where", ["key", "value", "every key"])
+def test_decode_batch_nan_entries(gpu, parts, where):
+    """A NaN in a history's keys (one entry, or all of them, so that no score of
+    a part is a number) or in its values makes that sequence's logits NaN and
+    leaves the others' bits, with histories of one part and of several, through
+    the one-launch paths and without them."""
+    model = parts["one"]
+    positions = [20, 20, 700, 700]
+    tokens = [5, 6, 7, 8]
+
+    def run(fused, spoiled):
+        g = torch.Generator(device="cuda").manual_seed(9)
+        seqs = [hip.Sequence(model, p + 1) for p in positions]
+        for i, (s, p) in enumerate(zip(seqs, positions)):
+            keys, values = s.tensors[3]
+            for t in (keys, values):
+                t[:p] = torch.randn(t[:p].shape, generator=g, device="cuda")
+            if i in spoiled:
+                if where == "every key":
+                    keys[:p] = float("nan")
+                else:
+                    (keys if where == "key" else values)[3, 1, 7] = float("nan")
+            s.struct.position = p
+        torch.cuda.synchronize()
+        out = torch.empty((len(positions), VOCAB), dtype=torch.float32, device="cuda")
+        gpu.set_fused_decode(fused)
+        try:
+            print("decode_batch NaN", where, fused, flush=True)
+            hip.decode_batch(gpu, model, tokens, seqs, out)
+            gpu.synchronize()
+        finally:
+            gpu.set_fused_decode(True)
+        return out.cpu().numpy()
+
+    clean = run(True, ())
+    for fused in (True, False):
+        got = run(fused, (1, 3))
+        assert np.isnan(got[[1, 3]]).all()
+        assert np.array_equal(got[[0, 2]].view(np.uint32), clean[[0, 2]].view(np.uint32))
+
+
 def test_fresh_sequences_batched_equal_decoded_alone(gpu, parts):
     """tests/model_batch_test.cpp:24-51: two new sequences decoded as one
     batch give the logits of each decoded alone, and both reach position 1.

@@ -571,7 +571,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
 // pairs. Both kernels, us, with their combines: 128 tokens at position 0 (8,000
 // pairs) 26 there, 34 here; 32 tokens at 500 and 16 at 1000 (16,000) 37 and
 // 36, 37 and 33 here; 256 tokens at 0 (33,000) 68 and 38; 512 at 3584 3065 and
-// 196.
+// 196. Fewer tokens than a block has were not compared and stay there.
 bool attention_chunk_takes(uint32_t position, uint32_t count) {
     return count >= kRowTokens && size_t(count) * (size_t(position) + count / 2u) >= 16384u;
 }

@@ -294,8 +294,11 @@ __device__ __forceinline__ float logit_of_key(uint32_t key) {
     return __uint_as_float((ascending & 0x80000000u) != 0u ? ascending ^ 0x80000000u : ~ascending);
 }
 
-// a / t, correctly rounded, from t's correctly rounded reciprocal: the first
-// product is within an ulp, and its exact remainder corrects it (Markstein).
+// a / t, correctly rounded, for a t of a float's 24 bits, from its rounded
+// reciprocal: the first product is off by less than two ulps, its remainder
+// a - q t fits a double, and the corrected sum is within 2^-52 of an ulp of
+// a / t before it is rounded, while a quotient by 24 bits comes no nearer than
+// 2^-25 of an ulp to the middle of two doubles.
 __device__ __forceinline__ double quotient(double a, double t, double inverse) {
     const double q = a * inverse;
     return fma(fma(-q, t, a), inverse, q);

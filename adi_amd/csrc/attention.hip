@@ -1357,8 +1357,10 @@ __global__ __launch_bounds__(kLinearHead) void k_linear_norm_gate(const float *r
                                                                   float *normalized, const float *qkv,
                                                                   float *convolution) {
 #pragma clang fp contract(off)
-    if (blockIdx.x == kValueHeads) {  // the grid's last column, after a chunk: the convolution state
-        for (uint32_t c = blockIdx.y * kLinearHead + threadIdx.x; c < kChannels; c += gridDim.y * kLinearHead) {
+    if (blockIdx.x >= kValueHeads) {  // the grid's last columns, after a chunk: the convolution state
+        const uint32_t block = (blockIdx.x - kValueHeads) * gridDim.y + blockIdx.y;
+        const uint32_t blocks = (gridDim.x - kValueHeads) * gridDim.y;
+        for (uint32_t c = block * kLinearHead + threadIdx.x; c < kChannels; c += blocks * kLinearHead) {
             shift_history(qkv, gridDim.y, convolution, c);
         }
         return;
@@ -1646,8 +1648,11 @@ void linear_attention_chunk(adi_hip_context *ctx, const adi_hip_linear_attention
                n, recurrent_state, recurrent_output + static_cast<size_t>(b0) * kValueSize);
     }
     // a chunk's state shifts here, where every token has read it, in blocks of
-    // its own (a launch for it alone took 4.7 us)
-    launch(ctx, "linear_norm_gate", k_linear_norm_gate, dim3(count > 1 ? kValueHeads + 1 : kValueHeads, count),
+    // its own (a launch for it alone took 4.7 us): one for each 128 channels, or
+    // as many as there are tokens (two blocks for all channels of two tokens
+    // took longer than the launch: 52.5 us a layer, 48.7 before)
+    const uint32_t shifts = count > 1 ? ceil_div(kChannels / kLinearHead, count) : 0u;
+    launch(ctx, "linear_norm_gate", k_linear_norm_gate, dim3(kValueHeads + shifts, count),
            dim3(kLinearHead), 0, static_cast<const float *>(recurrent_output), L->norm,
            static_cast<const float *>(gate), normalized, static_cast<const float *>(qkv), convolution_state);
     project_output(ctx, &L->output, normalized, count, outputs, norm_tail);

@@ -263,13 +263,14 @@ def test_linear_attention_prefill(gpu, oracle, tluts):
         close(drec.cpu().numpy(), rec, "recurrent state")
 
 
-@pytest.mark.parametrize("count", [2, 15, 16, 17, 33, 1025])
+@pytest.mark.parametrize("count", [2, 3, 15, 16, 17, 33, 64, 1025])
 def test_delta_chunk_edges(gpu, oracle, tluts, count):
     """The delta rule's chunk kernel at the edges of its sixteen-token stages
     and of its 1024-token launches, from a nonzero state: a dot of 128 products
     in another order differs by at most 128 * 2^-24 = 8e-6 of its magnitudes,
     and the decay keeps an error for a few tokens only, so 1e-4 of the largest
-    value bounds outputs and state."""
+    value bounds outputs and state. The convolution state is the last three
+    projected rows, shifted by as many blocks as the count leaves."""
     rng = syn.rng_for(65, count)
     layer = syn.linear_attention(rng, HIDDEN, tluts[1])
     d = hip.upload_linear_attention(gpu, layer, gpu.ne_codebook(tluts[1]))
@@ -284,6 +285,7 @@ def test_delta_chunk_edges(gpu, oracle, tluts, count):
                      for b in range(count)])
     assert max_rel_error(out.cpu().numpy(), want) <= 1e-4
     assert np.max(np.abs(drec.cpu().numpy() - rec)) <= 1e-4 * np.max(np.abs(rec))
+    assert np.max(np.abs(dconv.cpu().numpy() - conv)) <= 1e-4 * np.max(np.abs(conv))
 
 
 @pytest.mark.parametrize("full", [False, True])

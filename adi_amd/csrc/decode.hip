@@ -310,11 +310,11 @@ __device__ __forceinline__ double quotient(double a, double t, double inverse) {
 // a fixed tree; k_sample_rows adds the spans' sums in span order. A row with
 // a non-finite logit (a span index of 0xFFFFFFFF) gets sums of 0: the
 // sampler rejects it. Only bins that can matter take their tokens, every one of
-// them: tokens below p = (1 - top_p) / (1000 count) hold together less than a
-// thousandth of what top_p leaves out, so the bins behind the one of that p's
+// them: tokens below p = (1 - top_p) / (100 count) hold together less than a
+// hundredth of what top_p leaves out, so the bins behind the one of that p's
 // logit stay empty. An LDS atomic on one of the few bins of a normal tail waits
 // for its neighbours' (16 rows of 248,320 logits, temperature 0.7, top_p 0.9:
-// 36 us with every token binned, 25 us). A bin is taken whole because a bin is
+// 36 us with every token binned, 25 us from a thousandth on, 20 from here). A bin is taken whole because a bin is
 // an eighth of a binade of the logit and at a low temperature or a large logit
 // holds tokens of both kinds; the walks count a bin's tokens by these counts.
 __global__ __launch_bounds__(kArgmaxPartThreads) void k_expsum_parts(
@@ -1349,7 +1349,7 @@ int adi_hip_sample_rows(adi_hip_context *ctx, const float *logits, uint32_t rows
         // the log of the p below which a token cannot matter (top_p 1: -inf),
         // as a distance from the row's maximum
         const double reach = static_cast<double>(temperature) *
-                             std::log((1.0 - static_cast<double>(top_p)) * 1e-3 / static_cast<double>(count));
+                             std::log((1.0 - static_cast<double>(top_p)) * 1e-2 / static_cast<double>(count));
         launch(ctx, "expsum_parts", k_expsum_parts, dim3(parts, rows), dim3(kArgmaxPartThreads), 0,
                logits, count, span, static_cast<const float *>(part_value),
                static_cast<const uint32_t *>(part_index), temperature, reach, part_sum, top);

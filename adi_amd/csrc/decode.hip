@@ -616,9 +616,10 @@ struct CrossState {
 };
 
 // The bins of counts[kTopBins], masses[kTopBins] (plus `base` before them)
-// around a running sum of `target`, by a block of kSampleThreads.
-__device__ void cross_bins(const uint32_t *counts, const float *masses, double base, double target,
-                           CrossState &c, uint32_t *wave_count, double *wave_mass) {
+// around a running sum of `target`, by a block of kSampleThreads. Returns the
+// tokens in all bins.
+__device__ uint32_t cross_bins(const uint32_t *counts, const float *masses, double base, double target,
+                               CrossState &c, uint32_t *wave_count, double *wave_mass) {
     constexpr uint32_t kPer = kTopBins / kSampleThreads;
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     uint32_t n[kPer], own_n = 0;
@@ -719,6 +720,7 @@ __device__ void cross_bins(const uint32_t *counts, const float *masses, double b
         __syncthreads();
         place();
     }
+    return all;
 }
 
 // The tokens around a running sum of `target` over the row in (key, index)
@@ -731,7 +733,12 @@ __device__ uint32_t cross_window(const float *row, uint32_t count, double maximu
                                  double *wave_mass, double &before, bool &end) {
     const double inverse = 1.0 / temperature;
     const auto p_of = [&](float v) { return exp(quotient(static_cast<double>(v) - maximum, temperature, inverse)); };
-    cross_bins(row_counts, row_masses, 0.0, target, c, wave_count, wave_mass);
+    const uint32_t binned = cross_bins(row_counts, row_masses, 0.0, target, c, wave_count, wave_mass);
+    // (uniform) a range to the row's end holds the tokens of its empty bins too
+    // (a row that one window then decides: 391 us with its passes first, 349)
+    if (c.end != 0u && count - binned > kWindow) {
+        return 0;
+    }
     uint64_t first = static_cast<uint64_t>(c.lo) << kTopShift;
     uint64_t past = static_cast<uint64_t>(c.hi + 1u) << kTopShift;
     end = c.end != 0u;

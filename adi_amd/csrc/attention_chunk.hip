@@ -295,7 +295,9 @@ __global__ __launch_bounds__(kThreads, 2) void k_attention_chunk(ChunkArgs args)
             value_rows[(4u * wave + u) * kRow + lane] = entry(values, key0 + 4u * wave + u);
         }
         __syncthreads();
-        const uint32_t end = min(kKeys, min(args.position + wave_token + kWaveTokens, total) - key0);
+        // (a wave whose tokens all come before the tile has none)
+        const uint32_t past = min(args.position + wave_token + kWaveTokens, total);
+        const uint32_t end = past > key0 ? min(kKeys, past - key0) : 0u;
 #pragma unroll 1
         for (uint32_t k0 = 0; k0 < end && !__all(denominator != denominator); k0 += 4u) {
             float dot[4];
